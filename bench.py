@@ -45,8 +45,9 @@ BYTES_PER_CELL_UPDATE = 80  # read uold (5 x FP64) + write unew (5 x FP64)
 # Counters cannot be read while timing.  Each entry records the hash of the
 # kernel sources it was measured on (KERNEL_SOURCES); a build whose sources
 # hash differently reports null instead of a stale figure.
-KERNEL_SOURCES = ["ramses-cpp_amd/csrc/rh_hydro.hip", "ramses-cpp_amd/csrc/rh_physics.h",
-                  "ramses-cpp_amd/csrc/rh_kernels.h", "ramses-cpp_amd/Makefile"]
+KERNEL_SOURCES = ["ramses-cpp_amd/csrc/rh_hydro.hip", "ramses-cpp_amd/csrc/rh_godunov.hip",
+                  "ramses-cpp_amd/csrc/rh_fast.h", "ramses-cpp_amd/csrc/rh_device.h",
+                  "ramses-cpp_amd/csrc/rh_physics.h", "ramses-cpp_amd/csrc/rh_kernels.h", "ramses-cpp_amd/Makefile"]
 PROFILED = {
     (9, "hllc", 1, 2, "fp64"): {"sources": "aaea3b054087f57a", "traffic": 2172901455,
                                 "valu": {"busy": 0.761, "insts_per_cell": 5941.0, "courant_epilogue": True}},

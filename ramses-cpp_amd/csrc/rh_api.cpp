@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "rh_context.h"
+#include "rh_godunov.h"
 #include "rh_guard.h"
 #include "rh_kernels.h"
 #include "rh_tables.h"
@@ -288,7 +289,8 @@ double exact_inverse(double dx) {
 
 int variant_for(const rh_ctx* c, const rh::LevelDev& lv) {
     if (c->variant >= 0) return c->variant;
-    return (c->p.precision == RH_PREC_FP64 || lv.noct < AUTO_DIMS_MAX_OCTS) ? 6 : 2;
+    if (lv.noct < AUTO_DIMS_MAX_OCTS) return 6;
+    return c->p.precision == RH_PREC_FP64 && !rh::step_kernels_take(gas(c, c->p.gamma)) ? 6 : 2;
 }
 
 void drop_graph(StepGraph& g) {

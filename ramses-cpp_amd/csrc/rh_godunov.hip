@@ -1,0 +1,762 @@
+// rh_godunov.hip -- the Godunov update for ordinary states, one Riemann solver
+// per translation unit (RH_RIEMANN).
+//
+//   k_step_oct    one wave per 8 octs, the three dimensions one after another
+//   k_step_dims   three waves per 8 octs, one dimension each
+//
+// The eight cells of an oct sit in eight adjacent lanes, a lane's sibling
+// along dimension d is lane ^ (1 << d).  Both kernels run dim_pass, which
+// computes one dimension of a cell's update in the frame of rh_fast.h, and
+// general_cell for the octs of a wave in which some state is out of that
+// frame's range.
+//
+// Bound: the vector ALU.  An HLLC/MinMod update executes 3,046 VALU
+// instructions per cell in the FP64 form and 2,379 in the mixed form (the
+// kernels of rh_hydro.hip, which select each operand by a cell's place in its
+// oct, round every division separately and trace own and ghost states apart:
+// 5,941 and 3,958) at 81 % and 88 % VALU busy; HBM traffic is under a third of
+// what the memory delivers.  At 2^21 octs (256^3 cells) a launch takes 1.90 ms
+// in the FP64 form and 1.54 ms in the mixed form, against 3.48 and 2.09 ms;
+// at 512 octs 10.0 and 9.1 us against 13.6 and 12.9 us (k_step_dims).
+// Registers: three waves per SIMD (168 per lane) measured 1.90 ms against 2.04
+// at two in the FP64 form, 1.54 against 2.0 ms at four in the mixed form (which
+// then spills).
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "rh_device.h"
+#include "rh_fast.h"
+#include "rh_godunov.h"
+
+// Waves per SIMD asked for (registers per lane: 256 / 168 / 128 at 2 / 3 / 4).
+#ifndef RH_OCT_WAVES
+#define RH_OCT_WAVES 3
+#endif
+#ifndef RH_OCT_WAVES_F
+#define RH_OCT_WAVES_F 3
+#endif
+#ifndef RH_DIMS_WAVES
+#define RH_DIMS_WAVES 3
+#endif
+#ifndef RH_DIMS_WAVES_F
+#define RH_DIMS_WAVES_F 3
+#endif
+
+namespace rh {
+
+namespace {
+
+using fast::all_lanes;
+using fast::any_lane;
+using fast::Consts;
+using fast::flip;
+using fast::Slopes;
+
+// ---------------------------------------------------------------------------
+// General form of one cell's update: any finite or non-finite state, any mesh.
+// One lane does one cell on its own, with the routines of rh_physics.h.  It
+// is reached by waves that hold a state out of range or an oct that is its
+// own neighbour, so it is written for few registers and little code, not for
+// speed: one face flux at a time, the incoming ones recomputed in the order
+// they are applied.
+template <int R, bool MIXED>
+RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& gp, int p, int ic0, int cC, double dt,
+                         double dx, int f, bool incoming, double Fd[5]) {
+    using TC = typename std::conditional<MIXED, float, double>::type;
+    const Gas<double> gd{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1};
+    const Gas<TC> gc{(TC)gp.gamma, (TC)gp.gm1, (TC)gp.smalle, (TC)gp.smallp, (TC)(1.0 / gp.gm1)};
+    const TC dtc = (TC)dt;
+    const Len<TC, false> len{(TC)dx, TC(0)};
+    const int d = f >> 1, side = f & 1, b = 1 << d, par = (ic0 >> d) & 1;
+    // Rotated primitives of a cell; `fallback` where there is none.
+    auto prim = [&](int icell, const TC fallback[5], TC q[5]) {
+        if (icell > 0) {
+            double u[5];
+            load_u(m.uold, m.ncell, icell, u);
+            face_prim(u, q, gd, gc);
+            rotate(q, d);
+        } else {
+            copy5(fallback, q);
+        }
+    };
+    // The face state, on the side given, of a cell with left and right
+    // neighbours: its own (slope_type) or its ghost state (interpol_type).
+    auto state = [&](const TC a[5], const TC q[5], const TC c[5], bool own, bool upper, TC out[5]) {
+        TC dq[5], qm[5], qp[5], w = len.dx;
+        if (own) {
+            own_slopes(a, q, c, gp.slope_type, dtc, len, dq);
+        } else {
+            const Len<TC, false> lc = coarse(len);
+            w = lc.dx;
+            ghost_slopes(a, q, c, gp.interpol_type, lc, dq);
+        }
+        trace(q, dq, dtc, w, qm, qp, gc);
+        sel5(upper, qm, qp, out);
+    };
+    // The neighbour across the cell's oct face: in oct E, or a record.
+    const int E = lv.nbo[(size_t)(2 * d + par) * lv.noct + p];
+    int4 rc = make_int4(0, 0, 0, 0);
+    int X;
+    if (E >= 0) X = cell_id(m, lv.grid[E], ic0 ^ b);
+    else {
+        rc = lv.rec[-1 - E];
+        X = rc.x;
+    }
+    const int S = cell_id(m, lv.grid[p], ic0 ^ b);
+    const bool across = side == par;  // this face is the oct's face
+    // The cell N across the face, the cell beyond it, and whether N is there
+    // to solve with.
+    int beyond;
+    bool solve, reflux = false, bound = false;
+    if (!across) {
+        solve = (lv.leaf[p] >> (ic0 ^ b)) & 1;
+        const int E2 = lv.nbo[(size_t)(2 * d + 1 - par) * lv.noct + p];
+        beyond = E2 >= 0 ? cell_id(m, lv.grid[E2], ic0) : lv.rec[-1 - E2].x;
+    } else if (E >= 0) {
+        solve = (lv.leaf[E] >> (ic0 ^ b)) & 1;
+        beyond = cell_id(m, lv.grid[E], ic0);
+    } else {
+        solve = !incoming && !(rc.w & REC_REFINED_DEV);
+        bound = rc.w & REC_BOUNDARY_DEV;
+        reflux = solve && !bound;
+        beyond = side ? rc.z : rc.y;
+    }
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv) Fd[iv] = 0.0;
+    if (!solve) return;
+    TC qC[5], qN[5], qO[5], sC[5], sN[5];
+    prim(cC, qC, qC);
+    prim(across ? X : S, qC, qN);
+    prim(across ? S : X, qC, qO);
+    {
+        TC a[5], c[5];
+        sel5(side != 0, qO, qN, a);
+        sel5(side != 0, qN, qO, c);
+        state(a, qC, c, !incoming, side != 0, sC);
+    }
+    if (bound) {
+        double u[5];
+        load_u(m.uold, m.ncell, cC, u);
+#pragma unroll
+        for (int i = 1; i <= 3; ++i)
+            if (i == 1 + d) u[i] = u[i] * -1.0;
+        face_prim(u, qN, gd, gc);
+        rotate(qN, d);
+        TC dq[5] = {TC(0), TC(0), TC(0), TC(0), TC(0)}, other[5];
+        trace(qN, dq, dtc, len.dx, sN, other, gc);
+        sel5(side != 0, other, sN, sN);
+    } else {
+        // N's far neighbour and, on this side, the cell (a coarser N's own
+        // neighbour where N is a record).
+        TC far[5], a[5], c[5];
+        prim(beyond, qN, far);
+        if (reflux) prim(side ? rc.y : rc.z, qN, qC);
+        sel5(side != 0, qC, far, a);
+        sel5(side != 0, far, qC, c);
+        state(a, qN, c, incoming, side == 0, sN);
+    }
+    TC l[5], r[5], F[5];
+    sel5(side != 0, sC, sN, l);
+    sel5(side != 0, sN, sC, r);
+    solve_face<R, MIXED>(l, r, F, gc, gd);
+    rotate(F, d);
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv) Fd[iv] = (double)F[iv];
+    if (reflux) {
+        const int slot = lv.rec_slot[-1 - E] + face_slot(ic0, d);
+        const double sg = side ? -1.0 : 1.0;
+#pragma unroll
+        for (int iv = 0; iv < 5; ++iv) lv.slot_r[(size_t)slot * 5 + iv] = dt / dx * sg * Fd[iv] * 0.125;
+    }
+}
+
+template <int R, bool MIXED>
+RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, double u[5]) {
+    const MeshDev& m = a.m;
+    const LevelDev& lv = a.lv;
+    const GasParams& gp = a.gp;
+    const double* pre = a.pre;
+    double dt, dx = a.dx, inv_dx = a.inv_dx;
+    step_of(lv, p, a.d_dt, dt, dx, inv_dx);
+    const double dtdx = dt / dx;
+    double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, F[5];
+    long long kin[6];
+    incoming_keys(lv, p, ic0, lv.leaf[p], kin);
+    load_u(pre, m.ncell, cC, u);
+    const long long KOWN = ((long long)p * 8 + ic0) * 8 + 6;
+    int done = 0;
+    // Six own fluxes in face order, then the contributions in key order with
+    // the cell's own update among them.
+#pragma unroll 1
+    for (int it = 0; it < 13; ++it) {
+        asm volatile("" : "+v"(p), "+v"(ic0), "+v"(cC)::"memory");  // nothing is kept from one face to the next
+        int f = it;
+        if (it >= 6) {
+            long long best = (done & 64) ? KMAX : KOWN;
+            f = (done & 64) ? 7 : 6;
+#pragma unroll
+            for (int j = 0; j < 6; ++j) {
+                const bool take = !((done >> j) & 1) && kin[j] >= 0 && kin[j] < best;
+                best = take ? kin[j] : best;
+                f = take ? j : f;
+            }
+            if (f == 7) break;
+            done |= 1 << f;
+            if (f == 6) {
+                own_update(u, fs, dtdx, gp);
+                continue;
+            }
+        }
+        general_flux<R, MIXED>(m, lv, gp, p, ic0, cC, dt, dx, f, it >= 6, F);
+        if (it < 6) {
+            const double sg = (f & 1) ? -1.0 : 1.0;
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) fs[iv] = fs[iv] + sg * F[iv];
+        } else {
+            const double sdt = dtdx * ((f & 1) ? 1.0 : -1.0);
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] - sdt * F[iv] * 0.125;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+
+// Value of lane ^ (1 << D), through the LDS crossbar without an address.
+template <int D> RH_DEV int across_lanes(int x) { return __builtin_amdgcn_ds_swizzle(x, ((1 << D) << 10) | 0x1f); }
+template <int D> RH_DEV float sib(float x) { return __int_as_float(across_lanes<D>(__float_as_int(x))); }
+template <int D> RH_DEV double sib(double x) {
+    return __hiloint2double(across_lanes<D>(__double2hiint(x)), across_lanes<D>(__double2loint(x)));
+}
+
+// Component of a global state at position i of the rotated order.
+template <int D> constexpr int rot(int i) {
+    return i == 1 ? 1 + D : i == 2 ? (D == 1 ? 1 : 2) : i == 3 ? (D == 2 ? 1 : 3) : i;
+}
+
+// A cell's own fluxes of one dimension, in its frame and rotated order: Fe
+// through the oct's face, Fi towards its sibling.
+template <typename T> struct DimFlux {
+    T Fe[5], Fi[5];
+};
+
+// A wave's cells and constants.
+template <typename T> struct Cell {
+    int p, ic0, lm, cC;
+    bool leaf;
+    T q[5], y, c2;  // primitives in global order, recip(density), trace_c2
+};
+
+// A contribution to a cell is -((dtdx*sign)*F)*0.125 with the neighbour's flux
+// F in the global frame, added to the cell: k8*F in the cell's frame (k8 =
+// dtdx/8; the normal momentum's sign as given by s).  The FP64 form passes on
+// the product, the mixed form the FP32 flux, widened and multiplied where it
+// is added.
+RH_DEV double contribution(double F, double k8, int s) { return flip(k8, s) * F; }
+RH_DEV float contribution(float F, double, int s) { return flip(F, s); }
+RH_DEV double added(double w, double) { return w; }
+RH_DEV double added(float w, double k8) { return k8 * (double)w; }
+
+// One dimension of a cell's update: its own fluxes, the contributions of X
+// (into rows 5D+iv of s_x) and of S (ws), and key, the position of X's oct * 4
+// + D.  The external face comes first: what it needs of X is then dead, which
+// keeps the registers below 168 (three waves per SIMD).
+template <int R, typename T, bool EXACT, bool SHARED, int D>
+RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int interpol_type, const Consts<T>& k,
+                     const Cell<T>& c, double k8, bool& ok, DimFlux<T>& out, T ws[5], int& key, T (*s_x)[64],
+                     int t) {
+    const int b = 1 << D;
+    const bool par = (c.ic0 >> D) & 1;
+    const int sbit = par ? (int)0x80000000 : 0;
+    const int E = lv.nbo[(size_t)(2 * D + (par ? 1 : 0)) * lv.noct + c.p];
+    const int icS = c.ic0 ^ b;
+    int4 rc = make_int4(0, 0, 0, 0);
+    int Xcell, X2cell;
+    bool flux_x = true;  // X computes a flux through the shared face
+    if (E >= 0) {
+        const int g = lv.grid[E];
+        Xcell = cell_id(m, g, icS);
+        X2cell = cell_id(m, g, c.ic0);
+        flux_x = (lv.leaf[E] >> icS) & 1;
+    } else {
+        rc = lv.rec[-1 - E];
+        Xcell = rc.x;
+        X2cell = par ? rc.z : rc.y;
+        flux_x = false;
+    }
+    const bool special = any_lane(!flux_x);  // records or refined neighbours in this wave
+    const bool coarse = E < 0 && !(rc.w & (REC_REFINED_DEV | REC_BOUNDARY_DEV));
+    ok = ok && E != c.p;
+    key = (E >= 0 ? E * 4 : 0) + D;
+    if (special) {
+        // A boundary reads the cell's own state; a missing neighbour of a
+        // coarser cell the coarser cell's.
+        if (Xcell <= 0) Xcell = c.cC;
+        if (X2cell <= 0) X2cell = Xcell;
+    }
+    double u[5], w[5];
+    load_u(m.uold, m.ncell, Xcell, u);
+    load_u(m.uold, m.ncell, X2cell, w);
+
+    // The line C, S, X, X2 in the cell's frame; differences towards S.
+    T q[5], x[5], dl[5], dr[5], dx[5], g[5], yX, y2;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) q[i] = c.q[rot<D>(i)];
+    q[1] = flip(q[1], sbit);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        T s = sib<D>(q[i]);
+        if (i == 1) s = -s;
+        dr[i] = s - q[i];
+    }
+    fast::prim(u, g, yX, k, ok);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        x[i] = g[rot<D>(i)];
+        if (i == 1) x[i] = flip(x[i], sbit);
+        dl[i] = q[i] - x[i];
+    }
+    fast::prim(w, g, y2, k, ok);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        T z = g[rot<D>(i)];
+        if (i == 1) z = flip(z, sbit);
+        dx[i] = x[i] - z;
+    }
+    Slopes<T, SHARED> sc;
+    fast::slopes<T, SHARED, EXACT>(q, dl, dr, c.y, c.c2, slope_type, interpol_type, k, sc);
+
+    // X's states on the shared face, from X2, X and C (a coarser X's from its
+    // own neighbours; a boundary's is the cell's with the normal velocity
+    // reversed, without slopes).
+    T gx[5], om[5], l[5], F[5];
+    if (special) {
+        if (any_lane(coarse)) {
+            int far = par ? rc.y : rc.z;
+            if (!coarse || far <= 0) far = Xcell;
+            load_u(m.uold, m.ncell, far, u);
+            fast::prim(u, g, y2, k, ok);
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                T z = g[rot<D>(i)];
+                if (i == 1) z = flip(z, sbit);
+                dl[i] = coarse ? z - x[i] : dl[i];
+            }
+        }
+    }
+    {
+        Slopes<T, SHARED> sx;
+        fast::slopes<T, SHARED, EXACT>(x, dx, dl, yX, fast::trace_c2(x[0], x[4], yX, k), slope_type, interpol_type, k, sx);
+        fast::ghost_face<T, SHARED, EXACT>(x, sx, T(1.0), gx);
+        fast::own_face<T, SHARED, EXACT>(x, sx, T(1.0), om);
+    }
+    if (special) {
+        const bool bound = E < 0 && (rc.w & REC_BOUNDARY_DEV);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) gx[i] = bound ? (i == 1 ? -q[i] : q[i]) : gx[i];
+    }
+
+    // X's own flux through the shared face.
+    fast::ghost_face<T, SHARED, EXACT>(q, sc, T(-1.0), l);
+    fast::riemann<R>(om, l, F, k, par);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        const T wx = contribution(F[i], k8, i == 1 ? sbit : 0);
+        s_x[5 * D + rot<D>(i)][t] = special && !flux_x ? T(0) : wx;
+    }
+    // The cell's own.
+    fast::own_face<T, SHARED, EXACT>(q, sc, T(-1.0), l);
+    fast::riemann<R>(gx, l, out.Fe, k, par);
+    if (special) {
+        const bool none = E >= 0 ? !flux_x : (rc.w & REC_REFINED_DEV) != 0;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) out.Fe[i] = none ? T(0) : out.Fe[i];
+        if (coarse && c.leaf) {
+            const int slot = lv.rec_slot[-1 - E] + face_slot(c.ic0, D);
+#pragma unroll
+            for (int i = 0; i < 5; ++i)
+                lv.slot_r[(size_t)slot * 5 + rot<D>(i)] = flip(k8, i == 1 ? sbit : 0) * (double)out.Fe[i];
+        }
+    }
+
+    // Towards the sibling: the ghost state it sees on the shared face travels
+    // to it, its own comes here; then the fluxes change places.
+    T gs[5];
+    fast::ghost_face<T, SHARED, EXACT>(q, sc, T(1.0), gs);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) gs[i] = sib<D>(gs[i]);
+    gs[1] = -gs[1];
+    fast::own_face<T, SHARED, EXACT>(q, sc, T(1.0), l);
+    fast::riemann<R>(l, gs, out.Fi, k, par);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) F[i] = sib<D>(out.Fi[i]);
+    if (!all_lanes(c.lm == 0xff)) {
+        // A refined sibling: no flux through the face from either side.
+        const bool sib_leaf = (c.lm >> icS) & 1;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            out.Fi[i] = sib_leaf ? out.Fi[i] : T(0);
+            F[i] = sib_leaf ? F[i] : T(0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 5; ++i) ws[rot<D>(i)] = contribution(F[i], k8, i == 1 ? ~sbit & (int)0x80000000 : 0);
+}
+
+// The two own fluxes of a dimension as the reference's face loop adds them
+// (minus face, then plus face, signs included), in global order.
+template <int D, typename T> RH_DEV void own_terms(const DimFlux<T>& f, bool par, T first[5], T second[5]) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        const T e = f.Fe[i], n = f.Fi[i];
+        first[rot<D>(i)] = par ? (i == 1 ? n : -n) : e;
+        second[rot<D>(i)] = par ? (i == 1 ? -e : e) : -n;
+    }
+}
+// own_update() for a finite divisor range (density clamped to [1e-10, 1e6]).
+RH_DEV void own_update_fast(double u[5], const double fs[5], double dtdx, const GasParams& gp, double y_gm1) {
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] + dtdx * fs[iv];
+    const double d = sclamp(u[0], 1e-10, 1e6);
+    u[0] = d;
+    const double lim = d * 10.0, y = fast::recip(d);
+    double v2 = 0.0;
+#pragma unroll
+    for (int i = 1; i <= 3; ++i) {
+        u[i] = sclamp(u[i], -d * 10.0, lim);
+        const double v = fast::quot(u[i], d, y);
+        v2 = v2 + v * v;
+    }
+    const double ek = 0.5 * d * v2, least = fast::quot(d * 1e-10, gp.gm1, y_gm1);
+    if (u[4] - ek < least) u[4] = least + ek + 0.0;
+    u[4] = smin(u[4], d * 1e8);
+}
+
+// Wave speed sum of the Courant candidate, courant_cand_u() up to u_wave, for
+// a level without gravity; an out-of-range state takes the general divisions.
+RH_DEV double wave_speed(const double u[5], double gamma) {
+    const double d = smax(u[0], 1e-10);
+    const double s = (__builtin_fabs(u[1]) + __builtin_fabs(u[2])) + (__builtin_fabs(u[3]) + __builtin_fabs(u[4]));
+    double v[3], v2 = 0.0, c2;
+    if (all_lanes(s + d < 0x1p100)) {
+        const double y = fast::recip(d);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            v[i] = fast::quot(u[1 + i], d, y);
+            v2 = v2 + v[i] * v[i];
+        }
+        double pr = fast::mx((u[4] - 0.5 * d * v2) * (gamma - 1.0), d * 1e-10);
+        pr = fast::mn(pr, d * 1e2);
+        c2 = fast::mx(fast::quot(gamma * pr, d, y), 1e-10);
+        c2 = fast::root(c2);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            v[i] = u[1 + i] / d;
+            v2 = v2 + v[i] * v[i];
+        }
+        double pr = smax((u[4] - 0.5 * d * v2) * (gamma - 1.0), d * 1e-10);
+        pr = smin(pr, d * 1e2);
+        c2 = smax(gamma * pr / smax(d, 1e-10), 1e-20);
+        c2 = ssqrt(smax(c2, 1e-10));
+    }
+    double w = 3 * c2;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) w = w + sabs(v[i]);
+    return w;
+}
+
+// A wave's time step, cell width and constants, held in scalar registers.  All
+// its octs must be of one box; false when they are not, or when the time step
+// or the cell width is out of range.
+RH_DEV double uniform(double x) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+RH_DEV float uniform(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
+template <typename T>
+RH_DEV bool constants(const StepArgs& a, int p, double& dt, double& dx, Consts<T>& k) {
+    bool ok = true;
+    double inv_dx = a.inv_dx;
+    dx = a.dx;
+    if (a.lv.obox) {
+        const int mine = a.lv.obox[p], box = __builtin_amdgcn_readfirstlane(mine);
+        ok = mine == box;
+        dt = a.d_dt[box];
+        dx = a.lv.box_len[box];
+        inv_dx = a.lv.box_len[a.lv.nbox + box];
+    } else {
+        dt = *a.d_dt;
+    }
+    dt = uniform(dt);
+    dx = uniform(dx);
+    k.gamma = (T)a.gp.gamma;
+    k.gm1 = (T)a.gp.gm1;
+    k.smalle = (T)a.gp.smalle;
+    k.smallp = (T)a.gp.smallp;
+    k.dx = uniform((T)dx);
+    k.hdx = uniform(T(0.5) * k.dx);
+    k.hdt = uniform(T(0.5) * (T)dt);
+    const double dtdx = uniform(dt / dx);
+    if constexpr (sizeof(T) == 8) {
+        k.y_gm1 = uniform(fast::recip(a.gp.gm1));
+        k.inv = uniform(inv_dx != 0.0 ? inv_dx : fast::recip(dx));
+        return ok && dt >= 0x1p-100 && dtdx <= 0x1p20 && dx >= 0x1p-60 && dx <= 0x1p60;
+    } else {
+        k.y_gm1 = uniform((T)(1.0 / a.gp.gm1));
+        k.inv = uniform(fast::recip(k.dx));
+        return ok && dt >= 0x1p-50 && dtdx <= 0x1p20 && dx >= 0x1p-40 && dx <= 0x1p40;
+    }
+}
+
+// The ordered accumulation of a cell (processing order: position in the list,
+// then cell, then face).  An oct's neighbours across its faces come wholly
+// before or after it, so the order is: the X contributions of octs before
+// it by position, the siblings with a lower cell index (highest dimension
+// first), the cell itself, the siblings with a higher index, the X
+// contributions of octs after it.  wx: this lane's contributions in LDS, rows
+// 5d+iv from X of dimension d, rows 15+5d+iv from S of dimensions 0 and 1; ws2
+// those of dimension 2; key: position of the oct across * 4 + dimension.
+template <typename T>
+RH_DEV void apply(double u[5], const double fs[5], const T ws2[5], const T (*wx)[64], const int key[3], int p, int ic0,
+                  int t, double dtdx, const GasParams& gp, double y_gm1) {
+    const double k8 = dtdx * 0.125;
+    const int lo = min(min(key[0], key[1]), key[2]), hi = max(max(key[0], key[1]), key[2]);
+    const int k3[3] = {lo, key[0] ^ key[1] ^ key[2] ^ lo ^ hi, hi};
+    double x[3][5], ws[3][5];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int iv = 0; iv < 5; ++iv) {
+            x[j][iv] = added(wx[(k3[j] & 3) * 5 + iv][t], k8);
+            ws[j][iv] = added(j < 2 ? wx[15 + 5 * j + iv][t] : ws2[iv], k8);
+        }
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+        if (k3[j] < 4 * p)
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] + x[j][iv];
+#pragma unroll
+    for (int d = 2; d >= 0; --d)
+        if ((ic0 >> d) & 1)
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] + ws[d][iv];
+    own_update_fast(u, fs, dtdx, gp, y_gm1);
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        if (!((ic0 >> d) & 1))
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] + ws[d][iv];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+        if (k3[j] > 4 * p)
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] + x[j][iv];
+}
+
+// End of a cell's update: the new state into unew and, in the fused step, the
+// next step's Courant candidate (the state set_uold would copy).  Without
+// gravity a candidate falls monotonically with the cell's wave speed sum, each
+// operation rounding monotonically, so the wave takes the largest sum and
+// does the divisions once.
+RH_DEV void finish(const MeshDev& m, const LevelDev& lv, const GasParams& gp, const double u[5], bool leaf, int cC, int p,
+                   int pfirst, int t, double dx, double* cpart, unsigned long long* ckeys, double courant_factor) {
+    if (leaf) {
+#pragma unroll
+        for (int iv = 0; iv < 5; ++iv) m.unew[(size_t)iv * m.ncell + cC - 1] = u[iv];
+    }
+    if (!cpart && !ckeys) return;
+    const double s1 = ssqrt(1.0 + 2.0 * courant_factor * 1e-4) - 1.0;
+    const bool one_box = !ckeys || lv.obox[pfirst] == lv.obox[min(pfirst + 8, lv.noct) - 1];
+    double cand = __builtin_inf();
+    if (one_box && !m.f && s1 > 0.0) {
+        double w = leaf ? wave_speed(u, gp.gamma) : 0.0;
+        w = w > 0.0 ? w : 0.0;  // a NaN is skipped
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) w = fast::mx(w, __shfl_xor(w, off, 64));
+        if (w > 0.0) cand = (dx / w) * s1 / 1e-4;
+    } else {
+        if (leaf) cand = courant_cand_u(m, u, cC, dx, gp.gamma, courant_factor);
+        if (one_box) cand = wave_min(cand);
+    }
+    if (cpart) {
+        if (t == 0) cpart[blockIdx.x] = cand;
+    } else if (one_box) {
+        if (t == 0) atomicMin(&ckeys[lv.obox[pfirst]], dt_key(cand));
+    } else if (cand != __builtin_inf()) {
+        atomicMin(&ckeys[lv.obox[p]], dt_key(cand));
+    }
+}
+
+// This wave's cells: 8 octs of the list, lanes past its end on the last oct.
+template <typename T>
+RH_DEV void load_cell(const MeshDev& m, const LevelDev& lv, int praw, int t, const Consts<T>& k, Cell<T>& c, bool& ok) {
+    c.ic0 = t & 7;
+    c.p = min(praw, lv.noct - 1);
+    c.lm = lv.leaf[c.p];
+    c.leaf = praw < lv.noct && ((c.lm >> c.ic0) & 1);
+    c.cC = cell_id(m, lv.grid[c.p], c.ic0);
+    double u[5];
+    load_u(m.uold, m.ncell, c.cC, u);
+    fast::prim(u, c.q, c.y, k, ok);
+    c.c2 = fast::trace_c2(c.q[0], c.q[4], c.y, k);
+}
+
+template <int R, bool MIXED, bool EXACT, bool SHARED>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_OCT_WAVES_F : RH_OCT_WAVES, 8))) void k_step_oct(StepArgs a) {
+    using T = typename std::conditional<MIXED, float, double>::type;
+    __shared__ T s_x[25][64];
+    const MeshDev& m = a.m;
+    const LevelDev& lv = a.lv;
+    const int t = threadIdx.x;
+    const int praw = xcd_block(blockIdx.x, gridDim.x) * 8 + (t >> 3);
+    double dt, dx;
+    Consts<T> k;
+    Cell<T> c;
+    bool ok = constants(a, min(praw, lv.noct - 1), dt, dx, k);
+    load_cell(m, lv, praw, t, k, c, ok);
+    const double dtdx = uniform(dt / dx), k8 = uniform(dtdx * 0.125);
+    double fs[5], u[5];
+    T ws[5];
+    int key[3];
+    auto pass = [&](auto dc) {
+        constexpr int D = decltype(dc)::value;
+        DimFlux<T> f;
+        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, k8, ok, f, ws, key[D], s_x, t);
+        const bool par = (c.ic0 >> D) & 1;
+        if constexpr (D < 2)
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) s_x[15 + 5 * D + iv][t] = ws[iv];
+        if constexpr (D == 0) {
+            // From 0 the order of the two faces does not matter.
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                const double v = (double)f.Fe[i] - (double)f.Fi[i];
+                fs[rot<D>(i)] = i == 1 ? flip(v, par ? (int)0x80000000 : 0) : v;
+            }
+        } else {
+            T first[5], second[5];
+            own_terms<D>(f, par, first, second);
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) fs[iv] = (fs[iv] + (double)first[iv]) + (double)second[iv];
+        }
+    };
+    pass(std::integral_constant<int, 0>{});
+    pass(std::integral_constant<int, 1>{});
+    pass(std::integral_constant<int, 2>{});
+    load_u(a.pre, m.ncell, c.cC, u);
+    apply(u, fs, ws, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
+    if (!all_lanes(ok)) {
+        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, u);
+    }
+    finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a.cpart, a.ckeys, a.courant_factor);
+}
+
+// Own terms of one dimension, signs and order as own_terms().
+template <int D, typename T> RH_DEV void put_terms(const T first[5], const T second[5], T (*s_o)[64], int t) {
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv) {
+        s_o[10 * (D - 1) + iv][t] = first[iv];
+        s_o[10 * (D - 1) + 5 + iv][t] = second[iv];
+    }
+}
+
+template <int R, bool MIXED, bool EXACT, bool SHARED>
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_DIMS_WAVES_F : RH_DIMS_WAVES, 8))) void k_step_dims(StepArgs a) {
+    using T = typename std::conditional<MIXED, float, double>::type;
+    // Contributions of X and S per dimension, own terms of dimensions 1 and 2
+    // for the first wave, the oct across per dimension, range votes.
+    __shared__ T s_x[30][64];
+    __shared__ T s_o[20][64];
+    __shared__ int s_key[2][64];
+    __shared__ int s_bad[3];
+    const MeshDev& m = a.m;
+    const LevelDev& lv = a.lv;
+    const int t = threadIdx.x & 63;
+    const int d = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int praw = xcd_block(blockIdx.x, gridDim.x) * 8 + (t >> 3);
+    double dt, dx;
+    Consts<T> k;
+    Cell<T> c;
+    bool ok = constants(a, min(praw, lv.noct - 1), dt, dx, k);
+    load_cell(m, lv, praw, t, k, c, ok);
+    const double dtdx = uniform(dt / dx), k8 = uniform(dtdx * 0.125);
+    double fs[5];
+    int key[3];
+    auto pass = [&](auto dc) {
+        constexpr int D = decltype(dc)::value;
+        DimFlux<T> f;
+        T ws[5];
+        int kd;
+        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, k8, ok, f, ws, kd, s_x, t);
+        const bool par = (c.ic0 >> D) & 1;
+#pragma unroll
+        for (int iv = 0; iv < 5; ++iv) s_x[15 + 5 * D + iv][t] = ws[iv];
+        if constexpr (D == 0) {
+            key[0] = kd;
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                const double v = (double)f.Fe[i] - (double)f.Fi[i];
+                fs[rot<D>(i)] = i == 1 ? flip(v, par ? (int)0x80000000 : 0) : v;
+            }
+        } else {
+            s_key[D - 1][t] = kd;
+            T first[5], second[5];
+            own_terms<D>(f, par, first, second);
+            put_terms<D>(first, second, s_o, t);
+        }
+        const bool bad = !all_lanes(ok);  // every lane votes
+        if (t == 0) s_bad[D] = bad;
+    };
+    if (d == 0) pass(std::integral_constant<int, 0>{});
+    else if (d == 1) pass(std::integral_constant<int, 1>{});
+    else pass(std::integral_constant<int, 2>{});
+    __syncthreads();
+    if (d != 0) return;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        key[1 + j] = s_key[j][t];
+#pragma unroll
+        for (int iv = 0; iv < 5; ++iv) fs[iv] = (fs[iv] + (double)s_o[10 * j + iv][t]) + (double)s_o[10 * j + 5 + iv][t];
+    }
+    double u[5];
+    T ws2[5];
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv) ws2[iv] = s_x[25 + iv][t];
+    load_u(a.pre, m.ncell, c.cC, u);
+    apply(u, fs, ws2, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
+    if (s_bad[0] | s_bad[1] | s_bad[2]) {
+        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, u);
+    }
+    finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a.cpart, a.ckeys, a.courant_factor);
+}
+
+template <int R, bool MIXED, bool EXACT, bool SHARED>
+void launch_as(bool dims, const StepArgs& a, hipStream_t stream) {
+    const dim3 grid((a.lv.noct + 7) / 8);
+    if (dims) hipLaunchKernelGGL((k_step_dims<R, MIXED, EXACT, SHARED>), grid, dim3(192), 0, stream, a);
+    else hipLaunchKernelGGL((k_step_oct<R, MIXED, EXACT, SHARED>), grid, dim3(64), 0, stream, a);
+}
+template <int R, bool MIXED> void launch_prec(bool dims, const StepArgs& a, hipStream_t stream) {
+    const bool shared = a.gp.slope_type == 1 && a.gp.interpol_type == 1;
+    if (a.inv_dx != 0.0) {
+        if (shared) launch_as<R, MIXED, true, true>(dims, a, stream);
+        else launch_as<R, MIXED, true, false>(dims, a, stream);
+    } else {
+        if (shared) launch_as<R, MIXED, false, true>(dims, a, stream);
+        else launch_as<R, MIXED, false, false>(dims, a, stream);
+    }
+}
+
+}  // namespace
+
+template <int R> void launch_step(bool mixed, bool dims, const StepArgs& a, hipStream_t stream) {
+    if (mixed) launch_prec<R, true>(dims, a, stream);
+    else launch_prec<R, false>(dims, a, stream);
+}
+#ifndef RH_PROBE
+template void launch_step<RH_RIEMANN>(bool, bool, const StepArgs&, hipStream_t);
+#endif
+
+}  // namespace rh

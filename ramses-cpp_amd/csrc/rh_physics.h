@@ -406,8 +406,10 @@ template <typename T> RH_DEV void riemann_hllc(const T ql[5], const T qr[5], T f
     for (int i = 0; i < 5; ++i) flux[i] = fk[i] + sk * (us_v[i] - uk_v[i]);
 }
 
-// RiemannSolver.cpp:309-383 (nener=0)
-template <typename T> RH_DEV void riemann_acoustic(const T ql[5], const T qr[5], T flux[5], const Gas<T>& g) {
+// RiemannSolver.cpp:309-383 (nener=0).  mir: ql and qr are the two sides seen
+// in reverse, so a contact at rest belongs to the other one.
+template <typename T>
+RH_DEV void riemann_acoustic(const T ql[5], const T qr[5], T flux[5], const Gas<T>& g, bool mir = false) {
     const T smallr = T(1e-10);
     const T smallc = T(1e-10);
     T rl = smax(ql[0], smallr);
@@ -422,7 +424,7 @@ template <typename T> RH_DEV void riemann_acoustic(const T ql[5], const T qr[5],
     T wr = cr * rr;
     T pstar = dv((wr * pl + wl * pr) + wl * wr * (ul - ur), wl + wr + T(1e-20));
     T ustar = dv((wr * ur + wl * ul) + (pl - pr), wl + wr + T(1e-20));
-    T sgnm = (ustar >= T(0.0)) ? T(1.0) : T(-1.0);
+    T sgnm = (mir ? ustar > T(0.0) : ustar >= T(0.0)) ? T(1.0) : T(-1.0);
     bool lft = sgnm == T(1.0);
     T ro = lft ? rl : rr, uo = lft ? ul : ur, po = lft ? pl : pr, co = lft ? cl : cr;
     T rstar = ro + dv(pstar - po, smax(co * co, T(1e-20)));
@@ -579,7 +581,8 @@ RH_DEV void riemann_llf_f(const float ql[5], const float qr[5], float flux[5], c
     for (int i = 0; i < 5; ++i) flux[i] = 0.5f * (fl[i] + fr[i]) - 0.5f * a_max * (ur[i] - ul[i]);
 }
 
-RH_DEV void riemann_acoustic_f(const float ql[5], const float qr[5], float flux[5], const Gas<float>& gf) {
+RH_DEV void riemann_acoustic_f(const float ql[5], const float qr[5], float flux[5], const Gas<float>& gf,
+                               bool mir = false) {
     const float rl = smax(ql[0], 1e-10f), ul = ql[1], pl = smax(ql[4], rl * gf.smallp);
     const float rr = smax(qr[0], 1e-10f), ur = qr[1], pr = smax(qr[4], rr * gf.smallp);
     const float cl = ssqrt(cs2(rl, ql[4], gf)), cr = ssqrt(cs2(rr, qr[4], gf));
@@ -587,7 +590,7 @@ RH_DEV void riemann_acoustic_f(const float ql[5], const float qr[5], float flux[
     const float iw = __builtin_amdgcn_rcpf(wl + wr + 1e-20f);
     const float pstar = ((wr * pl + wl * pr) + wl * wr * (ul - ur)) * iw;
     const float ustar = ((wr * ur + wl * ul) + (pl - pr)) * iw;
-    const float sgnm = (ustar >= 0.0f) ? 1.0f : -1.0f;
+    const float sgnm = (mir ? ustar > 0.0f : ustar >= 0.0f) ? 1.0f : -1.0f;
     const bool lft = sgnm == 1.0f;
     const float ro = lft ? rl : rr, uo = lft ? ul : ur, po = lft ? pl : pr, co = lft ? cl : cr;
     float rstar = smax(ro + dv(pstar - po, smax(co * co, 1e-20f)), 1e-10f);
