@@ -84,8 +84,8 @@ int rh_timers_reset(rh_ctx* ctx);
  * the same cells.  All produce identical results.  -1 (the default of a new
  * context) chooses per level: 6 on levels of fewer than 16,384 octs and 2 on
  * larger ones (the fastest measured from 8 to 2^21 octs), except that the
- * FP64 form with slope_type 4 or 5, or with gamma - 1 outside [2^-10, 64],
- * takes 6 on every level.  rh_autotune and
+ * FP64 form with slope_type 4 or 5, with gamma - 1 outside [2^-10, 64] or on
+ * a mesh of more than 2^29 cells takes 6 on every level.  rh_autotune and
  * rh_set_kernel_variant fix one variant for every level of the context;
  * rh_get_kernel_variant reports -1 while the default is in use. */
 #define RH_KERNEL_VARIANTS 7

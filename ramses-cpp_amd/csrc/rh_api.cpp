@@ -290,7 +290,7 @@ double exact_inverse(double dx) {
 int variant_for(const rh_ctx* c, const rh::LevelDev& lv) {
     if (c->variant >= 0) return c->variant;
     if (lv.noct < AUTO_DIMS_MAX_OCTS) return 6;
-    return c->p.precision == RH_PREC_FP64 && !rh::step_kernels_take(gas(c, c->p.gamma)) ? 6 : 2;
+    return c->p.precision == RH_PREC_FP64 && !rh::step_kernels_take(gas(c, c->p.gamma), c->mesh.ncell) ? 6 : 2;
 }
 
 void drop_graph(StepGraph& g) {

@@ -7,9 +7,10 @@
 // reads; a wave with a state outside takes the general code) means finite and
 // far from overflow and underflow, so that
 //   * a quotient needs neither the scaling nor the fix-up of the IEEE
-//     division sequence: reciprocal, two Newton steps, one corrected product
-//     -- the same steps on the same operands, 8 instructions instead of 12,
-//     and quotients by one divisor share its reciprocal (3 each);
+//     division sequence: a reciprocal refined to the last bit (4 instructions)
+//     and a product corrected by its exact remainder (3), which rounds
+//     correctly as IEEE division does; quotients by one divisor share its
+//     reciprocal;
 //   * a square root needs no scaling (11 instructions instead of 18);
 //   * no operand of a minimum or maximum is a NaN, so v_min/v_max replace
 //     compare-and-select pairs (3 instructions for a double);
@@ -47,14 +48,13 @@ RH_DEV float fm(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 RH_DEV double signed_as(double a, double s) { return __builtin_copysign(a, s); }
 RH_DEV float signed_as(float a, float s) { return __builtin_copysignf(a, s); }
 
-// Reciprocal as the IEEE division sequence refines it, and a quotient by a
-// divisor whose reciprocal is known (float: the hardware reciprocal, as dv()).
+// Reciprocal (the hardware's, good to 2^-23 at least, times 1 + e + e^2 with
+// its error e: 2^-69 before the last rounding), and a quotient by a divisor
+// whose reciprocal is known (float: the hardware reciprocal, as dv()).
 RH_DEV double recip(double b) {
     const double y = __builtin_amdgcn_rcp(b);
     const double e = fm(-b, y, 1.0);
-    const double y1 = fm(y, e, y);
-    const double e1 = fm(-b, y1, 1.0);
-    return fm(y1, e1, y1);
+    return fm(y, fm(e, e, e), y);
 }
 RH_DEV float recip(float b) { return __builtin_amdgcn_rcpf(b); }
 RH_DEV double quot(double a, double b, double y) {
@@ -95,7 +95,7 @@ template <typename T> struct Consts {
 RH_DEV double e_int(double p, const Consts<double>& k) { return quot(p, k.gm1, k.y_gm1); }
 RH_DEV float e_int(float p, const Consts<float>& k) { return p * k.y_gm1; }
 
-// Bounds of a state in range.  Within them, and with dt/dx <= 2^20, dt >=
+// Upper bound of a state in range (prim).  Within its bounds, and with dt/dx <= 2^20, dt >=
 // 2^-100 (mixed 2^-50), dx in [2^-60, 2^60] and gamma - 1 in [2^-10, 64], no
 // FP64 intermediate of the update exceeds 1e290 and none that is rounded
 // falls below the normal numbers; the smallest difference of two velocities
@@ -103,50 +103,47 @@ RH_DEV float e_int(float p, const Consts<float>& k) { return p * k.y_gm1; }
 constexpr double RANGE_HI = 0x1p50;
 
 // Conservative -> primitive (the operations of ctoprim); y = recip(density).
-// ok is cleared when the state is out of range: s covers |density|, the
-// kinetic and the total specific energy before its floor (a NaN or an
-// infinity in any component reaches s); a velocity other than 0 must not be
-// tiny, and in FP32 neither must density and pressure (frexp's exponent of 0
-// is 0, so a zero velocity passes).
+// ok is cleared when the state is out of range: below the floors (density and
+// internal specific energy t of at least RANGE_LO; then no floor of ctoprim or
+// of the trace's sound speed applies either), too large (s covers the density,
+// t and twice the kinetic specific energy; a NaN or an infinity in any
+// component reaches s), or with a velocity that is tiny but not 0 (frexp's
+// exponent of 0 is 0, so a zero velocity passes).
 RH_DEV void prim(const double u[5], double q[5], double& y, const Consts<double>& k, bool& ok) {
-    const double d = mx(u[0], 1e-10);
-    y = recip(d);
-    const double o = unit_quot(d, y);
-    q[0] = d;
+    y = recip(u[0]);
+    const double o = unit_quot(u[0], y);
+    q[0] = u[0];
     q[1] = u[1] * o;
     q[2] = u[2] * o;
     q[3] = u[3] * o;
-    const double ek = (0.5 * q[1] * q[1] + 0.5 * q[2] * q[2]) + 0.5 * q[3] * q[3];
-    const double t = u[4] * o - ek;
-    q[4] = k.gm1 * d * mx(t, k.smalle);
-    const double s = (ek + __builtin_fabs(t)) + __builtin_fabs(u[0]);
+    const double v2 = (q[1] * q[1] + q[2] * q[2]) + q[3] * q[3];
+    const double t = fm(-0.5, v2, u[4] * o);
+    q[4] = k.gm1 * u[0] * t;
+    const double s = (v2 + t) + u[0];
     const int least = min(min(__builtin_amdgcn_frexp_exp(q[1]), __builtin_amdgcn_frexp_exp(q[2])),
                           __builtin_amdgcn_frexp_exp(q[3]));
-    ok = ok && s < RANGE_HI && least > -200;
+    ok = ok & (s < RANGE_HI) & (mn(u[0], t) >= 1e-10) & (least > -200);
 }
 RH_DEV void prim(const double ud[5], float q[5], float& y, const Consts<float>& k, bool& ok) {
     float u[5];
 #pragma unroll
     for (int i = 0; i < 5; ++i) u[i] = (float)ud[i];
-    const float d = mx(u[0], 1e-10f);
-    y = recip(d);
-    q[0] = d;
+    y = recip(u[0]);
+    q[0] = u[0];
     q[1] = u[1] * y;
     q[2] = u[2] * y;
     q[3] = u[3] * y;
-    const float ek = (0.5f * q[1] * q[1] + 0.5f * q[2] * q[2]) + 0.5f * q[3] * q[3];
-    const float t = u[4] * y - ek;
-    q[4] = k.gm1 * d * mx(t, k.smalle);
-    const float s = (ek + __builtin_fabsf(t)) + __builtin_fabsf(u[0]);
+    const float v2 = (q[1] * q[1] + q[2] * q[2]) + q[3] * q[3];
+    const float t = fm(-0.5f, v2, u[4] * y);
+    q[4] = k.gm1 * u[0] * t;
+    const float s = (v2 + t) + u[0];
     const int least = min(min(__builtin_amdgcn_frexp_expf(q[1]), __builtin_amdgcn_frexp_expf(q[2])),
                           __builtin_amdgcn_frexp_expf(q[3]));
-    ok = ok && s < (float)RANGE_HI && least > -45 && mn(d, q[4]) > 0x1p-45f;
+    ok = ok & (s < (float)RANGE_HI) & (mn(u[0], t) >= 0x1p-20f) & (least > -45);
 }
 
-// Sound speed squared of a trace (pressure floored at r*1e-20).
-template <typename T> RH_DEV T trace_c2(T r, T p, T y, const Consts<T>& k) {
-    return mx(quot(k.gamma * mx(p, r * T(1e-20)), r, y), T(1e-20));
-}
+// Sound speed squared of a trace (its floors: see prim).
+template <typename T> RH_DEV T trace_c2(T r, T p, T y, const Consts<T>& k) { return quot(k.gamma * p, r, y); }
 
 // minmod(a, b): the smaller of two differences of one sign, else 0.
 RH_DEV double minmod(double a, double b) { return mx(mn(a, b), mn(mx(a, b), 0.0)); }
@@ -181,15 +178,17 @@ RH_DEV void half_sources(const T q[5], T y, T c2, T dr, T du, T dp, const Consts
 }
 
 // One face state of a cell: q + s*A (+ B on density, normal velocity and
-// pressure), A given as the factor times the vector h it is exact in.
+// pressure), A given as the factor times the vector h it is exact in.  least
+// keeps the smallest face density: the trace's density floor (the cell's own
+// density below 1e-10) is left to the general form.
 template <typename T>
-RH_DEV void face(const T q[5], const T h[5], T f, const T B[3], T fb, T out[5]) {
+RH_DEV void face(const T q[5], const T h[5], T f, const T B[3], T fb, T out[5], T& least) {
     out[0] = fm(fb, B[0], fm(f, h[0], q[0]));
     out[1] = fm(fb, B[1], fm(f, h[1], q[1]));
     out[2] = fm(f, h[2], q[2]);
     out[3] = fm(f, h[3], q[3]);
     out[4] = fm(fb, B[2], fm(f, h[4], q[4]));
-    if (out[0] < T(1e-10)) out[0] = q[0];
+    least = mn(least, out[0]);
 }
 
 // Slopes of a cell in a form its face states are built from: own state on
@@ -239,19 +238,19 @@ RH_DEV void slopes(const T q[5], const T a[5], const T b[5], T y, T c2, int slop
 }
 // up: +1 for the face towards S, -1 for the face towards X.
 template <typename T, bool SHARED, bool EXACT>
-RH_DEV void own_face(const T q[5], const Slopes<T, SHARED>& s, T up, T out[5]) {
-    face(q, s.ho, up * (EXACT ? T(0.5) : T(1.0)), s.Bo, T(1.0), out);
+RH_DEV void own_face(const T q[5], const Slopes<T, SHARED>& s, T up, T out[5], T& least) {
+    face(q, s.ho, up * (EXACT ? T(0.5) : T(1.0)), s.Bo, T(1.0), out, least);
 }
 template <typename T, bool SHARED, bool EXACT>
-RH_DEV void ghost_face(const T q[5], const Slopes<T, SHARED>& s, T up, T out[5]) {
-    if constexpr (SHARED) face(q, s.ho, up * (EXACT ? T(0.25) : T(0.5)), s.Bo, T(0.25), out);
-    else face(q, s.hg, up * (EXACT ? T(0.5) : T(1.0)), s.Bg, T(1.0), out);
+RH_DEV void ghost_face(const T q[5], const Slopes<T, SHARED>& s, T up, T out[5], T& least) {
+    if constexpr (SHARED) face(q, s.ho, up * (EXACT ? T(0.25) : T(0.5)), s.Bo, T(0.25), out, least);
+    else face(q, s.hg, up * (EXACT ? T(0.5) : T(1.0)), s.Bg, T(1.0), out, least);
 }
 
 // Physical flux and total energy of a face state.
 template <typename T> RH_DEV void flux_of(const T q[5], T f[5], T& mu, T& E, const Consts<T>& k) {
     mu = q[0] * q[1];
-    E = T(0.5) * q[0] * ((q[1] * q[1] + q[2] * q[2]) + q[3] * q[3]) + e_int(q[4], k);
+    E = fm(T(0.5), q[0] * ((q[1] * q[1] + q[2] * q[2]) + q[3] * q[3]), e_int(q[4], k));
     f[0] = mu;
     f[1] = mu * q[1] + q[4];
     f[2] = mu * q[2];
@@ -259,47 +258,48 @@ template <typename T> RH_DEV void flux_of(const T q[5], T f[5], T& mu, T& E, con
     f[4] = (E + q[4]) * q[1];
 }
 template <typename T> RH_DEV T face_c2(const T q[5], const Consts<T>& k) {
-    return mx(quot(k.gamma * q[4], q[0], recip(q[0])), T(1e-20));
+    return quot(k.gamma * q[4], q[0], recip(q[0]));
 }
 
-// riemann_hllc.  Face densities are at least 1e-10 (face()), so its floors
-// on them are left out; only the larger sound speed is used and the square
-// root is monotone, so one root serves.  The side of the contact, and the
-// side whose physical flux is the answer where both signals run one way, are
-// one choice; there the star term is multiplied by 0 instead of branching.
-template <typename T> RH_DEV void hllc(const T l[5], const T r[5], T F[5], const Consts<T>& k, bool mir) {
-    const T pl = mx(l[4], l[0] * k.smallp), pr = mx(r[4], r[0] * k.smallp);
-    const T c = root(mx(face_c2(l, k), face_c2(r, k)));
+// riemann_hllc.  Its floors on densities, pressures, sound speeds and the
+// contact speed are left to the general form: ok is cleared where one would
+// apply (a pressure below density*smallp has a squared sound speed of at most
+// 1e-20).  Only the larger sound speed is used and the square root is
+// monotone, so one root serves.  The side of the contact, and the side whose
+// physical flux is the answer where both signals run one way, are one choice;
+// there the star term is multiplied by 0 instead of branching.
+template <typename T> RH_DEV void hllc(const T l[5], const T r[5], T F[5], const Consts<T>& k, bool mir, bool& ok) {
+    const T c2l = face_c2(l, k), c2r = face_c2(r, k);
+    const T c = root(mx(c2l, c2r));
     const T sl = mn(l[1], r[1]) - c, sr = mx(l[1], r[1]) + c;
     const T al = l[0] * (l[1] - sl), ar = r[0] * (sr - r[1]);
     const T div = ar + al;
     const T yd = recip(div);
-    T us = quot((ar * r[1] + al * l[1]) + (pl - pr), div, yd);
-    us = mx(T(-1e6), mn(T(1e6), us));
-    const T ps = mx(quot((ar * pl + al * pr) + al * ar * (l[1] - r[1]), div, yd), T(0.0));
+    const T us = quot((ar * r[1] + al * l[1]) + (l[4] - r[4]), div, yd);
+    const T ps = mx(quot((ar * l[4] + al * r[4]) + al * ar * (l[1] - r[1]), div, yd), T(0.0));
+    ok = ok & (mn(c2l, c2r) >= T(2e-20)) & (sabs(us) <= T(1e6));
     const bool pass_l = sl > T(0.0), pass_r = sr < T(0.0);
-    const T tie = sizeof(T) == 8 ? T(-4.9406564584124654e-324) : T(-1.4012984643e-45f);
-    const bool left = pass_l || (!pass_r && us > (mir ? tie : T(0.0)));
+    const bool left = pass_l | (!pass_r & ((us > T(0.0)) | (mir & (us == T(0.0)))));
     T q[5];
 #pragma unroll
     for (int i = 0; i < 5; ++i) q[i] = left ? l[i] : r[i];
-    const T pk = left ? pl : pr, sk = left ? sl : sr;
-    const T raw = sk - us;
-    const T den = left ? mn(raw, T(-1e-10)) : mx(raw, T(1e-10));
+    const T sk = left ? sl : sr;
+    const int away = left ? 0 : (int)0x80000000;  // den is negative on the left side, positive on the right
+    const T den = flip(mn(flip(sk - us, away), T(-1e-10)), away);
     const T ye = recip(den);
     const T dsu = sk - q[1];
     const T rs = quot(q[0] * dsu, den, ye);
     T f[5], mu, E;
     flux_of(q, f, mu, E, k);
-    const T Es = quot((dsu * E - pk * q[1]) + ps * us, den, ye);
-    const T s = (pass_l || pass_r) ? T(0.0) : sk;
+    const T Es = quot((dsu * E - q[4] * q[1]) + ps * us, den, ye);
+    const T s = (pass_l | pass_r) ? T(0.0) : sk;
     F[0] = f[0] + s * (rs - q[0]);
     F[1] = f[1] + s * (rs * us - mu);
     F[2] = f[2] + s * (rs * q[2] - q[0] * q[2]);
     F[3] = f[3] + s * (rs * q[3] - q[0] * q[3]);
     F[4] = f[4] + s * (Es - E);
-    const bool cold = div < T(1e-5) && !pass_l && !pass_r;
-    if (any_lane(cold)) {
+    const bool cold = (div < T(1e-5)) & !pass_l & !pass_r;
+    if (__builtin_expect(any_lane(cold), 0)) {
         T fl[5], fr[5];
         flux_of(l, fl, mu, E, k);
         flux_of(r, fr, mu, E, k);
@@ -313,7 +313,7 @@ template <typename T> RH_DEV void llf(const T l[5], const T r[5], T F[5], const 
     T fl[5], fr[5], ml, mr, El, Er;
     flux_of(l, fl, ml, El, k);
     flux_of(r, fr, mr, Er, k);
-    const T cl = root(face_c2(l, k)), cr = root(face_c2(r, k));
+    const T cl = root(mx(face_c2(l, k), T(1e-20))), cr = root(mx(face_c2(r, k), T(1e-20)));
     const T am = T(0.5) * mx(sabs(l[1]) + cl, sabs(r[1]) + cr);
     F[0] = T(0.5) * (fl[0] + fr[0]) - am * (r[0] - l[0]);
     F[1] = T(0.5) * (fl[1] + fr[1]) - am * (mr - ml);
@@ -325,7 +325,7 @@ template <typename T> RH_DEV void hll(const T l[5], const T r[5], T F[5], const 
     T fl[5], fr[5], ml, mr, El, Er;
     flux_of(l, fl, ml, El, k);
     flux_of(r, fr, mr, Er, k);
-    const T cl = root(face_c2(l, k)), cr = root(face_c2(r, k));
+    const T cl = root(mx(face_c2(l, k), T(1e-20))), cr = root(mx(face_c2(r, k), T(1e-20)));
     const T sl = mn(T(0.0), mn(l[1] - cl, r[1] - cr)), sr = mx(T(0.0), mx(l[1] + cl, r[1] + cr));
     const T w = sr - sl, i = unit_quot(w, recip(w)), ss = sr * sl;
     F[0] = ((sr * fl[0] - sl * fr[0]) + ss * (r[0] - l[0])) * i;
@@ -344,8 +344,9 @@ RH_DEV void acoustic(const float l[5], const float r[5], float F[5], const Const
     riemann_acoustic_f(l, r, F, Gas<float>{k.gamma, k.gm1, k.smalle, k.smallp, k.y_gm1}, mir);
 }
 
-template <int R, typename T> RH_DEV void riemann(const T l[5], const T r[5], T F[5], const Consts<T>& k, bool mir) {
-    if constexpr (R == 2) hllc(l, r, F, k, mir);
+template <int R, typename T>
+RH_DEV void riemann(const T l[5], const T r[5], T F[5], const Consts<T>& k, bool mir, bool& ok) {
+    if constexpr (R == 2) hllc(l, r, F, k, mir, ok);
     else if constexpr (R == 1) hll(l, r, F, k);
     else if constexpr (R == 4) acoustic(l, r, F, k, mir);
     else llf(l, r, F, k);

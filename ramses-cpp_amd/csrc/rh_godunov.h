@@ -24,10 +24,11 @@ struct StepArgs {
 
 // Whether the update runs in these kernels for a configuration: their slope
 // limiters are those symmetric under a reversed axis (types 4 and 5, whose two
-// sides are weighted by the sign of the velocity, are not), and their range
-// analysis holds for gamma - 1 in [2^-10, 64].
-inline bool step_kernels_take(const GasParams& gp) {
-    return gp.slope_type != 4 && gp.slope_type != 5 && gp.gm1 >= 0x1p-10 && gp.gm1 <= 64.0;
+// sides are weighted by the sign of the velocity, are not), their range
+// analysis holds for gamma - 1 in [2^-10, 64], and they address a state
+// component, and the six neighbour tables of a level, by 32-bit byte offsets.
+inline bool step_kernels_take(const GasParams& gp, int ncell) {
+    return gp.slope_type != 4 && gp.slope_type != 5 && gp.gm1 >= 0x1p-10 && gp.gm1 <= 64.0 && ncell <= (1 << 29);
 }
 
 // dims: three waves per 8 octs, one per dimension; else one wave.

@@ -10,17 +10,18 @@
 // general_cell for the octs of a wave in which some state is out of that
 // frame's range.
 //
-// Bound: the vector ALU.  An HLLC/MinMod update executes 3,046 VALU
-// instructions per cell in the FP64 form and 2,379 in the mixed form (the
-// kernels of rh_hydro.hip, which select each operand by a cell's place in its
-// oct, round every division separately and trace own and ghost states apart:
-// 5,941 and 3,958) at 81 % and 88 % VALU busy; HBM traffic is under a third of
-// what the memory delivers.  At 2^21 octs (256^3 cells) a launch takes 1.90 ms
-// in the FP64 form and 1.54 ms in the mixed form, against 3.48 and 2.09 ms;
-// at 512 octs 10.0 and 9.1 us against 13.6 and 12.9 us (k_step_dims).
-// Registers: three waves per SIMD (168 per lane) measured 1.90 ms against 2.04
-// at two in the FP64 form, 1.54 against 2.0 ms at four in the mixed form (which
-// then spills).
+// Bound: the vector ALU, 91-96 % busy.  An HLLC/MinMod update executes about
+// 2,750 VALU instructions per cell in the FP64 form and 2,150 in the mixed form
+// (the kernels of rh_hydro.hip, which select each operand by a cell's place in
+// its oct, round every division separately and trace own and ghost states
+// apart: 5,941 and 3,958); HBM traffic is a quarter of what the memory
+// delivers.  At 2^21 octs (256^3 cells) a launch takes 1.75-1.80 ms in the FP64
+// form and 1.47-1.50 ms in the mixed form, against 3.48 and 2.09 ms; at 512
+// octs 10.0 and 9.1 us against 13.6 and 12.9 us (k_step_dims).
+// Registers: three waves per SIMD (168 per lane).  Two waves took 2.04 ms
+// against 1.90 (FP64, an earlier order of the code), four waves 1.61 against
+// 1.49 (mixed, 24 bytes spilled): a spill is written through to memory for
+// every wave, so what the update keeps per lane is arranged to need none.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -59,42 +60,84 @@ using fast::Slopes;
 // is reached by waves that hold a state out of range or an oct that is its
 // own neighbour, so it is written for few registers and little code, not for
 // speed: one face flux at a time, the incoming ones recomputed in the order
-// they are applied.
-template <int R, bool MIXED>
+// they are applied, states and slopes in the lane's column of LDS (w, the 25
+// rows that the ordinary form keeps its contributions in) and the components
+// taken one after another.  Held to the registers of the ordinary form it
+// costs waves in range nothing; with its states in registers the kernel
+// spilled in the ordinary form too (FP64 1.77 ms per launch at 2^21 octs
+// became 1.84).
+template <typename T> struct Rows {
+    T (*w)[64];
+    int t;
+    RH_DEV T& operator()(int row) const { return w[row][t]; }
+};
+constexpr int ROW_C = 0, ROW_N = 5, ROW_O = 10, ROW_SC = 15, ROW_SN = 20;
+
+// Rotated primitives of a cell into rows `to`; rows `fallback` where there is
+// no cell.
+template <typename T>
+RH_DEV void general_prim(const MeshDev& m, const GasParams& gp, const Gas<T>& gc, int icell, int d, int fallback, int to,
+                         const Rows<T>& W) {
+    if (icell > 0) {
+        const Gas<double> gd{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1};
+        double u[5];
+        T q[5];
+        load_u(m.uold, m.ncell, icell, u);
+        face_prim(u, q, gd, gc);
+        rotate(q, d);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) W(to + i) = q[i];
+    } else {
+#pragma unroll 1
+        for (int i = 0; i < 5; ++i) W(to + i) = W(fallback + i);
+    }
+}
+
+// The face state, on the side given (upper: towards the right neighbour), of
+// the cell in rows q with left and right neighbours in rows a and c, into rows
+// `to`: its own (slope_type) or its ghost state (interpol_type).  The
+// operations of own_slopes / ghost_slopes and trace.
+template <typename T>
+RH_DEV void general_state(const GasParams& gp, const Gas<T>& gc, T dt, T dx, int a, int q, int c, bool own, bool upper,
+                          int to, const Rows<T>& W) {
+    const Len<T, false> lo{dx, T(0)};
+    const Len<T, false> len = own ? lo : coarse(lo);
+    const int st = gp.slope_type;
+    const T nu = over(W(q + 1) * dt, lo);
+#pragma unroll 1
+    for (int i = 0; i < 5; ++i) {
+        const T qa = W(a + i), qb = W(q + i), qc = W(c + i);
+        T lim;
+        if (own) lim = (st == 0 || ((st == 5 || st == 6) && i != 0)) ? T(0.0) : limiter(qa, qb, qc, st, nu);
+        else lim = ghost_limiter(qb - qa, qc - qb, gp.interpol_type);
+        W(to + i) = (own && (st == 0 || ((st == 5 || st == 6) && i != 0))) ? T(0.0) : over(lim, len);
+    }
+    const T dr = W(to), du = W(to + 1), dp = W(to + 4);
+    const T r = smax(W(q), T(1e-10)), u = W(q + 1);
+    const T c2 = cs2(r, smax(W(q + 4), r * T(1e-20)), gc);
+    const T s0 = -u * dr - du * r, s1 = -u * du - dv(dp, r), s4 = -u * dp - du * r * c2;
+    const T hdx = T(0.5) * len.dx, hdt = T(0.5) * dt;
+#pragma unroll 1
+    for (int i = 0; i < 5; ++i) {
+        const T step = hdx * W(to + i), src = i == 0 ? s0 : i == 1 ? s1 : i == 4 ? s4 : T(0);
+        T v = (upper ? W(q + i) + step : W(q + i) - step) + hdt * src;
+        if (i == 0 && v < T(1e-10)) v = r;
+        W(to + i) = v;
+    }
+}
+
+// One face flux of a cell, its own through face f or, incoming, the one its
+// neighbour there computes for the shared face (0 where there is none).
+template <int R, bool MIXED, typename T>
 RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& gp, int p, int ic0, int cC, double dt,
-                         double dx, int f, bool incoming, double Fd[5]) {
-    using TC = typename std::conditional<MIXED, float, double>::type;
-    const Gas<double> gd{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1};
-    const Gas<TC> gc{(TC)gp.gamma, (TC)gp.gm1, (TC)gp.smalle, (TC)gp.smallp, (TC)(1.0 / gp.gm1)};
-    const TC dtc = (TC)dt;
-    const Len<TC, false> len{(TC)dx, TC(0)};
+                         double dx, int f, bool incoming, const Rows<T>& W, double Fd[5]) {
+    const Gas<T> gc{(T)gp.gamma, (T)gp.gm1, (T)gp.smalle, (T)gp.smallp, (T)(1.0 / gp.gm1)};
+    const T dtc = (T)dt, dxc = (T)dx;
     const int d = f >> 1, side = f & 1, b = 1 << d, par = (ic0 >> d) & 1;
-    // Rotated primitives of a cell; `fallback` where there is none.
-    auto prim = [&](int icell, const TC fallback[5], TC q[5]) {
-        if (icell > 0) {
-            double u[5];
-            load_u(m.uold, m.ncell, icell, u);
-            face_prim(u, q, gd, gc);
-            rotate(q, d);
-        } else {
-            copy5(fallback, q);
-        }
-    };
-    // The face state, on the side given, of a cell with left and right
-    // neighbours: its own (slope_type) or its ghost state (interpol_type).
-    auto state = [&](const TC a[5], const TC q[5], const TC c[5], bool own, bool upper, TC out[5]) {
-        TC dq[5], qm[5], qp[5], w = len.dx;
-        if (own) {
-            own_slopes(a, q, c, gp.slope_type, dtc, len, dq);
-        } else {
-            const Len<TC, false> lc = coarse(len);
-            w = lc.dx;
-            ghost_slopes(a, q, c, gp.interpol_type, lc, dq);
-        }
-        trace(q, dq, dtc, w, qm, qp, gc);
-        sel5(upper, qm, qp, out);
-    };
-    // The neighbour across the cell's oct face: in oct E, or a record.
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv) Fd[iv] = 0.0;
+    // The neighbour X across the cell's oct face (in oct E, or a record) and
+    // its sibling S.
     const int E = lv.nbo[(size_t)(2 * d + par) * lv.noct + p];
     int4 rc = make_int4(0, 0, 0, 0);
     int X;
@@ -105,7 +148,7 @@ RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& 
     }
     const int S = cell_id(m, lv.grid[p], ic0 ^ b);
     const bool across = side == par;  // this face is the oct's face
-    // The cell N across the face, the cell beyond it, and whether N is there
+    // The cell beyond the neighbour N across the face, and whether N is there
     // to solve with.
     int beyond;
     bool solve, reflux = false, bound = false;
@@ -122,44 +165,41 @@ RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& 
         reflux = solve && !bound;
         beyond = side ? rc.z : rc.y;
     }
-#pragma unroll
-    for (int iv = 0; iv < 5; ++iv) Fd[iv] = 0.0;
     if (!solve) return;
-    TC qC[5], qN[5], qO[5], sC[5], sN[5];
-    prim(cC, qC, qC);
-    prim(across ? X : S, qC, qN);
-    prim(across ? S : X, qC, qO);
-    {
-        TC a[5], c[5];
-        sel5(side != 0, qO, qN, a);
-        sel5(side != 0, qN, qO, c);
-        state(a, qC, c, !incoming, side != 0, sC);
-    }
+    general_prim(m, gp, gc, cC, d, ROW_C, ROW_C, W);
+    general_prim(m, gp, gc, across ? X : S, d, ROW_C, ROW_N, W);
+    general_prim(m, gp, gc, across ? S : X, d, ROW_C, ROW_O, W);
+    general_state(gp, gc, dtc, dxc, side ? ROW_O : ROW_N, ROW_C, side ? ROW_N : ROW_O, !incoming, side != 0, ROW_SC, W);
     if (bound) {
+        // The cell's own state with the normal momentum reversed, traced
+        // without slopes.
+        const Gas<double> gd{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1};
         double u[5];
         load_u(m.uold, m.ncell, cC, u);
 #pragma unroll
         for (int i = 1; i <= 3; ++i)
             if (i == 1 + d) u[i] = u[i] * -1.0;
-        face_prim(u, qN, gd, gc);
-        rotate(qN, d);
-        TC dq[5] = {TC(0), TC(0), TC(0), TC(0), TC(0)}, other[5];
-        trace(qN, dq, dtc, len.dx, sN, other, gc);
-        sel5(side != 0, other, sN, sN);
+        T q[5], qm[5], qp[5], dq[5] = {T(0), T(0), T(0), T(0), T(0)};
+        face_prim(u, q, gd, gc);
+        rotate(q, d);
+        trace(q, dq, dtc, dxc, qm, qp, gc);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) W(ROW_SN + i) = side ? qp[i] : qm[i];
     } else {
         // N's far neighbour and, on this side, the cell (a coarser N's own
         // neighbour where N is a record).
-        TC far[5], a[5], c[5];
-        prim(beyond, qN, far);
-        if (reflux) prim(side ? rc.y : rc.z, qN, qC);
-        sel5(side != 0, qC, far, a);
-        sel5(side != 0, far, qC, c);
-        state(a, qN, c, incoming, side == 0, sN);
+        general_prim(m, gp, gc, beyond, d, ROW_N, ROW_O, W);
+        if (reflux) general_prim(m, gp, gc, side ? rc.y : rc.z, d, ROW_N, ROW_C, W);
+        general_state(gp, gc, dtc, dxc, side ? ROW_C : ROW_O, ROW_N, side ? ROW_O : ROW_C, incoming, side == 0, ROW_SN,
+                      W);
     }
-    TC l[5], r[5], F[5];
-    sel5(side != 0, sC, sN, l);
-    sel5(side != 0, sN, sC, r);
-    solve_face<R, MIXED>(l, r, F, gc, gd);
+    T l[5], r[5], F[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        l[i] = W((side ? ROW_SC : ROW_SN) + i);
+        r[i] = W((side ? ROW_SN : ROW_SC) + i);
+    }
+    solve_face<R, MIXED>(l, r, F, gc, Gas<double>{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1});
     rotate(F, d);
 #pragma unroll
     for (int iv = 0; iv < 5; ++iv) Fd[iv] = (double)F[iv];
@@ -171,19 +211,17 @@ RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& 
     }
 }
 
-template <int R, bool MIXED>
-RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, double u[5]) {
+template <int R, bool MIXED, typename T>
+RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, T (*w)[64], int t, double u[5]) {
     const MeshDev& m = a.m;
     const LevelDev& lv = a.lv;
     const GasParams& gp = a.gp;
-    const double* pre = a.pre;
+    const Rows<T> W{w, t};
     double dt, dx = a.dx, inv_dx = a.inv_dx;
     step_of(lv, p, a.d_dt, dt, dx, inv_dx);
     const double dtdx = dt / dx;
     double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, F[5];
-    long long kin[6];
-    incoming_keys(lv, p, ic0, lv.leaf[p], kin);
-    load_u(pre, m.ncell, cC, u);
+    load_u(a.pre, m.ncell, cC, u);
     const long long KOWN = ((long long)p * 8 + ic0) * 8 + 6;
     int done = 0;
     // Six own fluxes in face order, then the contributions in key order with
@@ -193,6 +231,8 @@ RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, double u[5])
         asm volatile("" : "+v"(p), "+v"(ic0), "+v"(cC)::"memory");  // nothing is kept from one face to the next
         int f = it;
         if (it >= 6) {
+            long long kin[6];
+            incoming_keys(lv, p, ic0, lv.leaf[p], kin);
             long long best = (done & 64) ? KMAX : KOWN;
             f = (done & 64) ? 7 : 6;
 #pragma unroll
@@ -208,7 +248,7 @@ RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, double u[5])
                 continue;
             }
         }
-        general_flux<R, MIXED>(m, lv, gp, p, ic0, cC, dt, dx, f, it >= 6, F);
+        general_flux<R, MIXED>(m, lv, gp, p, ic0, cC, dt, dx, f, it >= 6, W, F);
         if (it < 6) {
             const double sg = (f & 1) ? -1.0 : 1.0;
 #pragma unroll
@@ -222,6 +262,32 @@ RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, double u[5])
 }
 
 // ---------------------------------------------------------------------------
+
+// Element i of an array at a byte offset that fits 32 bits (step_kernels_take):
+// the base stays in scalar registers and the lane's part of the address is one
+// 32-bit value, shared by the five components of a state.  The empty asm keeps
+// the compiler from adding the two up in 64 bits per component.
+template <typename E> using GlobalPtr = __attribute__((address_space(1))) E*;
+template <typename E> RH_DEV GlobalPtr<E> scalar_base(E* p) {
+    GlobalPtr<E> g = (GlobalPtr<E>)p;
+    asm("" : "+s"(g));
+    return g;
+}
+template <typename E> RH_DEV E at(const E* base, unsigned i) {
+    return *(GlobalPtr<const E>)((GlobalPtr<const char>)scalar_base(base) + i * (unsigned)sizeof(E));
+}
+RH_DEV void load5(const MeshDev& m, const double* u, int icell, double out[5]) {
+    const unsigned off = ((unsigned)icell - 1u) * 8u;
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv)
+        out[iv] = *(GlobalPtr<const double>)((GlobalPtr<const char>)scalar_base(u + (size_t)iv * m.ncell) + off);
+}
+RH_DEV void store5(const MeshDev& m, double* u, int icell, const double v[5]) {
+    const unsigned off = ((unsigned)icell - 1u) * 8u;
+#pragma unroll
+    for (int iv = 0; iv < 5; ++iv)
+        *(GlobalPtr<double>)((GlobalPtr<char>)scalar_base(u + (size_t)iv * m.ncell) + off) = v[iv];
+}
 
 // Value of lane ^ (1 << D), through the LDS crossbar without an address.
 template <int D> RH_DEV int across_lanes(int x) { return __builtin_amdgcn_ds_swizzle(x, ((1 << D) << 10) | 0x1f); }
@@ -258,46 +324,52 @@ RH_DEV float contribution(float F, double, int s) { return flip(F, s); }
 RH_DEV double added(double w, double) { return w; }
 RH_DEV double added(float w, double k8) { return k8 * (double)w; }
 
+// A cell's neighbours across its oct's face along a dimension: the oct E there
+// (or a record code), the cells X and X2 whose states the line reads, and
+// whether X computes a flux through the shared face.
+struct Across {
+    int E, X, X2;
+    bool flux_x;
+};
+template <int D, typename T> RH_DEV int oct_across(const LevelDev& lv, const Cell<T>& c) {
+    return at(lv.nbo, (2u * D + ((c.ic0 >> D) & 1u)) * (unsigned)lv.noct + (unsigned)c.p);
+}
+template <int D, typename T> RH_DEV Across across(const MeshDev& m, const LevelDev& lv, const Cell<T>& c, int E) {
+    Across n{E, c.cC, c.cC, false};
+    if (E >= 0) {
+        const int g = at(lv.grid, E), icS = c.ic0 ^ (1 << D);
+        n.X = cell_id(m, g, icS);
+        n.X2 = cell_id(m, g, c.ic0);
+        n.flux_x = (at(lv.leaf, E) >> icS) & 1;
+    } else {
+        // A boundary reads the cell's own state, a missing neighbour of a
+        // coarser cell the coarser cell's.
+        const int4 rc = lv.rec[-1 - E];
+        const int far = ((c.ic0 >> D) & 1) ? rc.z : rc.y;
+        if (rc.x > 0) n.X = rc.x;
+        n.X2 = far > 0 ? far : n.X;
+    }
+    return n;
+}
+
 // One dimension of a cell's update: its own fluxes, the contributions of X
-// (into rows 5D+iv of s_x) and of S (ws), and key, the position of X's oct * 4
-// + D.  The external face comes first: what it needs of X is then dead, which
-// keeps the registers below 168 (three waves per SIMD).
-template <int R, typename T, bool EXACT, bool SHARED, int D>
+// (into rows 5D+iv of s_x) and of S (ws).  u, w: the states of X and X2.  The
+// external face comes first: what it needs of X is then dead, which keeps the
+// registers below 168 (three waves per SIMD); next() issues the loads of the
+// next dimension's states after the last solve (before it they cost 20 more
+// registers and the kernel spills; without it, 1.83 ms against 1.77).
+template <int R, typename T, bool EXACT, bool SHARED, int D, typename Next>
 RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int interpol_type, const Consts<T>& k,
-                     const Cell<T>& c, double k8, bool& ok, DimFlux<T>& out, T ws[5], int& key, T (*s_x)[64],
-                     int t) {
-    const int b = 1 << D;
+                     const Cell<T>& c, const Across& n, double u[5], const double w[5], double k8, bool& ok,
+                     DimFlux<T>& out, T ws[5], T (*s_x)[64], int t, Next next) {
     const bool par = (c.ic0 >> D) & 1;
     const int sbit = par ? (int)0x80000000 : 0;
-    const int E = lv.nbo[(size_t)(2 * D + (par ? 1 : 0)) * lv.noct + c.p];
-    const int icS = c.ic0 ^ b;
+    const int E = n.E;
+    const bool special = any_lane(!n.flux_x);  // records or refined neighbours in this wave
     int4 rc = make_int4(0, 0, 0, 0);
-    int Xcell, X2cell;
-    bool flux_x = true;  // X computes a flux through the shared face
-    if (E >= 0) {
-        const int g = lv.grid[E];
-        Xcell = cell_id(m, g, icS);
-        X2cell = cell_id(m, g, c.ic0);
-        flux_x = (lv.leaf[E] >> icS) & 1;
-    } else {
-        rc = lv.rec[-1 - E];
-        Xcell = rc.x;
-        X2cell = par ? rc.z : rc.y;
-        flux_x = false;
-    }
-    const bool special = any_lane(!flux_x);  // records or refined neighbours in this wave
+    if (special && E < 0) rc = lv.rec[-1 - E];
     const bool coarse = E < 0 && !(rc.w & (REC_REFINED_DEV | REC_BOUNDARY_DEV));
-    ok = ok && E != c.p;
-    key = (E >= 0 ? E * 4 : 0) + D;
-    if (special) {
-        // A boundary reads the cell's own state; a missing neighbour of a
-        // coarser cell the coarser cell's.
-        if (Xcell <= 0) Xcell = c.cC;
-        if (X2cell <= 0) X2cell = Xcell;
-    }
-    double u[5], w[5];
-    load_u(m.uold, m.ncell, Xcell, u);
-    load_u(m.uold, m.ncell, X2cell, w);
+    ok = ok & (E != c.p);
 
     // The line C, S, X, X2 in the cell's frame; differences towards S.
     T q[5], x[5], dl[5], dr[5], dx[5], g[5], yX, y2;
@@ -330,12 +402,12 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
     // X's states on the shared face, from X2, X and C (a coarser X's from its
     // own neighbours; a boundary's is the cell's with the normal velocity
     // reversed, without slopes).
-    T gx[5], om[5], l[5], F[5];
-    if (special) {
-        if (any_lane(coarse)) {
+    T gx[5], om[5], l[5], F[5], least = q[0];
+    if (__builtin_expect(special, 0)) {
+        if (__builtin_expect(any_lane(coarse), 0)) {
             int far = par ? rc.y : rc.z;
-            if (!coarse || far <= 0) far = Xcell;
-            load_u(m.uold, m.ncell, far, u);
+            if (!coarse || far <= 0) far = n.X;
+            load5(m, m.uold, far, u);
             fast::prim(u, g, y2, k, ok);
 #pragma unroll
             for (int i = 0; i < 5; ++i) {
@@ -348,30 +420,30 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
     {
         Slopes<T, SHARED> sx;
         fast::slopes<T, SHARED, EXACT>(x, dx, dl, yX, fast::trace_c2(x[0], x[4], yX, k), slope_type, interpol_type, k, sx);
-        fast::ghost_face<T, SHARED, EXACT>(x, sx, T(1.0), gx);
-        fast::own_face<T, SHARED, EXACT>(x, sx, T(1.0), om);
+        fast::ghost_face<T, SHARED, EXACT>(x, sx, T(1.0), gx, least);
+        fast::own_face<T, SHARED, EXACT>(x, sx, T(1.0), om, least);
     }
-    if (special) {
+    if (__builtin_expect(special, 0)) {
         const bool bound = E < 0 && (rc.w & REC_BOUNDARY_DEV);
 #pragma unroll
         for (int i = 0; i < 5; ++i) gx[i] = bound ? (i == 1 ? -q[i] : q[i]) : gx[i];
     }
 
     // X's own flux through the shared face.
-    fast::ghost_face<T, SHARED, EXACT>(q, sc, T(-1.0), l);
-    fast::riemann<R>(om, l, F, k, par);
+    fast::ghost_face<T, SHARED, EXACT>(q, sc, T(-1.0), l, least);
+    fast::riemann<R>(om, l, F, k, par, ok);
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        const T wx = contribution(F[i], k8, i == 1 ? sbit : 0);
-        s_x[5 * D + rot<D>(i)][t] = special && !flux_x ? T(0) : wx;
-    }
+    for (int i = 0; i < 5; ++i) s_x[5 * D + rot<D>(i)][t] = contribution(F[i], k8, i == 1 ? sbit : 0);
     // The cell's own.
-    fast::own_face<T, SHARED, EXACT>(q, sc, T(-1.0), l);
-    fast::riemann<R>(gx, l, out.Fe, k, par);
-    if (special) {
-        const bool none = E >= 0 ? !flux_x : (rc.w & REC_REFINED_DEV) != 0;
+    fast::own_face<T, SHARED, EXACT>(q, sc, T(-1.0), l, least);
+    fast::riemann<R>(gx, l, out.Fe, k, par, ok);
+    if (__builtin_expect(special, 0)) {
+        const bool none = E >= 0 ? !n.flux_x : (rc.w & REC_REFINED_DEV) != 0;
 #pragma unroll
-        for (int i = 0; i < 5; ++i) out.Fe[i] = none ? T(0) : out.Fe[i];
+        for (int i = 0; i < 5; ++i) {
+            out.Fe[i] = none ? T(0) : out.Fe[i];
+            if (!n.flux_x) s_x[5 * D + i][t] = T(0);
+        }
         if (coarse && c.leaf) {
             const int slot = lv.rec_slot[-1 - E] + face_slot(c.ic0, D);
 #pragma unroll
@@ -383,17 +455,19 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
     // Towards the sibling: the ghost state it sees on the shared face travels
     // to it, its own comes here; then the fluxes change places.
     T gs[5];
-    fast::ghost_face<T, SHARED, EXACT>(q, sc, T(1.0), gs);
+    fast::ghost_face<T, SHARED, EXACT>(q, sc, T(1.0), gs, least);
 #pragma unroll
     for (int i = 0; i < 5; ++i) gs[i] = sib<D>(gs[i]);
     gs[1] = -gs[1];
-    fast::own_face<T, SHARED, EXACT>(q, sc, T(1.0), l);
-    fast::riemann<R>(l, gs, out.Fi, k, par);
+    fast::own_face<T, SHARED, EXACT>(q, sc, T(1.0), l, least);
+    ok = ok & (least >= T(1e-10));
+    fast::riemann<R>(l, gs, out.Fi, k, par, ok);
+    next();
 #pragma unroll
     for (int i = 0; i < 5; ++i) F[i] = sib<D>(out.Fi[i]);
-    if (!all_lanes(c.lm == 0xff)) {
+    if (__builtin_expect(!all_lanes(c.lm == 0xff), 0)) {
         // A refined sibling: no flux through the face from either side.
-        const bool sib_leaf = (c.lm >> icS) & 1;
+        const bool sib_leaf = (c.lm >> (c.ic0 ^ (1 << D))) & 1;
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
             out.Fi[i] = sib_leaf ? out.Fi[i] : T(0);
@@ -404,33 +478,48 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
     for (int i = 0; i < 5; ++i) ws[rot<D>(i)] = contribution(F[i], k8, i == 1 ? ~sbit & (int)0x80000000 : 0);
 }
 
-// The two own fluxes of a dimension as the reference's face loop adds them
-// (minus face, then plus face, signs included), in global order.
-template <int D, typename T> RH_DEV void own_terms(const DimFlux<T>& f, bool par, T first[5], T second[5]) {
+// Adds a dimension's own fluxes as the reference's face loop does: the minus
+// face, then minus the plus face, in global order.
+template <int D, typename T> RH_DEV void add_own(double fs[5], const DimFlux<T>& f, bool par) {
+    if (par) {
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        const T e = f.Fe[i], n = f.Fi[i];
-        first[rot<D>(i)] = par ? (i == 1 ? n : -n) : e;
-        second[rot<D>(i)] = par ? (i == 1 ? -e : e) : -n;
+        for (int i = 0; i < 5; ++i) {
+            const double e = (double)f.Fe[i], n = (double)f.Fi[i];
+            double& s = fs[rot<D>(i)];
+            s = i == 1 ? (s + n) - e : (s - n) + e;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            double& s = fs[rot<D>(i)];
+            s = (s + (double)f.Fe[i]) - (double)f.Fi[i];
+        }
     }
 }
-// own_update() for a finite divisor range (density clamped to [1e-10, 1e6]).
+
+// own_update() for finite values (applies_to() votes on the state it starts
+// from; what is added to it is bounded by the range of the states).
 RH_DEV void own_update_fast(double u[5], const double fs[5], double dtdx, const GasParams& gp, double y_gm1) {
 #pragma unroll
     for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] + dtdx * fs[iv];
-    const double d = sclamp(u[0], 1e-10, 1e6);
+    const double d = fast::mn(fast::mx(u[0], 1e-10), 1e6);
     u[0] = d;
     const double lim = d * 10.0, y = fast::recip(d);
     double v2 = 0.0;
 #pragma unroll
     for (int i = 1; i <= 3; ++i) {
-        u[i] = sclamp(u[i], -d * 10.0, lim);
+        u[i] = fast::mn(fast::mx(u[i], -lim), lim);
         const double v = fast::quot(u[i], d, y);
         v2 = v2 + v * v;
     }
-    const double ek = 0.5 * d * v2, least = fast::quot(d * 1e-10, gp.gm1, y_gm1);
-    if (u[4] - ek < least) u[4] = least + ek + 0.0;
-    u[4] = smin(u[4], d * 1e8);
+    const double dv2 = d * v2, least = fast::quot(d * 1e-10, gp.gm1, y_gm1);
+    if (__builtin_fma(-0.5, dv2, u[4]) < least) u[4] = __builtin_fma(0.5, dv2, least);
+    u[4] = fast::mn(u[4], d * 1e8);
+}
+// Whether the state an update starts from is finite and no larger than 2^100
+// (it is uold's, already in range, except where a caller has changed unew).
+RH_DEV bool applies_to(const double u[5]) {
+    return ((fabs(u[0]) + fabs(u[1])) + (fabs(u[2]) + fabs(u[3]))) + fabs(u[4]) < 0x1p100;
 }
 
 // Wave speed sum of the Courant candidate, courant_cand_u() up to u_wave, for
@@ -446,7 +535,7 @@ RH_DEV double wave_speed(const double u[5], double gamma) {
             v[i] = fast::quot(u[1 + i], d, y);
             v2 = v2 + v[i] * v[i];
         }
-        double pr = fast::mx((u[4] - 0.5 * d * v2) * (gamma - 1.0), d * 1e-10);
+        double pr = fast::mx(__builtin_fma(-0.5, d * v2, u[4]) * (gamma - 1.0), d * 1e-10);
         pr = fast::mn(pr, d * 1e2);
         c2 = fast::mx(fast::quot(gamma * pr, d, y), 1e-10);
         c2 = fast::root(c2);
@@ -517,7 +606,8 @@ RH_DEV bool constants(const StepArgs& a, int p, double& dt, double& dx, Consts<T
 // first), the cell itself, the siblings with a higher index, the X
 // contributions of octs after it.  wx: this lane's contributions in LDS, rows
 // 5d+iv from X of dimension d, rows 15+5d+iv from S of dimensions 0 and 1; ws2
-// those of dimension 2; key: position of the oct across * 4 + dimension.
+// those of dimension 2; key: position of the oct across * 4 + dimension (a
+// record's is negative and its contribution 0).
 template <typename T>
 RH_DEV void apply(double u[5], const double fs[5], const T ws2[5], const T (*wx)[64], const int key[3], int p, int ic0,
                   int t, double dtdx, const GasParams& gp, double y_gm1) {
@@ -562,10 +652,7 @@ RH_DEV void apply(double u[5], const double fs[5], const T ws2[5], const T (*wx)
 // does the divisions once.
 RH_DEV void finish(const MeshDev& m, const LevelDev& lv, const GasParams& gp, const double u[5], bool leaf, int cC, int p,
                    int pfirst, int t, double dx, double* cpart, unsigned long long* ckeys, double courant_factor) {
-    if (leaf) {
-#pragma unroll
-        for (int iv = 0; iv < 5; ++iv) m.unew[(size_t)iv * m.ncell + cC - 1] = u[iv];
-    }
+    if (leaf) store5(m, m.unew, cC, u);
     if (!cpart && !ckeys) return;
     const double s1 = ssqrt(1.0 + 2.0 * courant_factor * 1e-4) - 1.0;
     const bool one_box = !ckeys || lv.obox[pfirst] == lv.obox[min(pfirst + 8, lv.noct) - 1];
@@ -594,11 +681,11 @@ template <typename T>
 RH_DEV void load_cell(const MeshDev& m, const LevelDev& lv, int praw, int t, const Consts<T>& k, Cell<T>& c, bool& ok) {
     c.ic0 = t & 7;
     c.p = min(praw, lv.noct - 1);
-    c.lm = lv.leaf[c.p];
+    c.lm = at(lv.leaf, c.p);
     c.leaf = praw < lv.noct && ((c.lm >> c.ic0) & 1);
-    c.cC = cell_id(m, lv.grid[c.p], c.ic0);
+    c.cC = cell_id(m, at(lv.grid, c.p), c.ic0);
     double u[5];
-    load_u(m.uold, m.ncell, c.cC, u);
+    load5(m, m.uold, c.cC, u);
     fast::prim(u, c.q, c.y, k, ok);
     c.c2 = fast::trace_c2(c.q[0], c.q[4], c.y, k);
 }
@@ -617,13 +704,27 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
     bool ok = constants(a, min(praw, lv.noct - 1), dt, dx, k);
     load_cell(m, lv, praw, t, k, c, ok);
     const double dtdx = uniform(dt / dx), k8 = uniform(dtdx * 0.125);
-    double fs[5], u[5];
+    const int E0 = oct_across<0>(lv, c), E1 = oct_across<1>(lv, c), E2 = oct_across<2>(lv, c);
+    const Across n[3] = {across<0>(m, lv, c, E0), across<1>(m, lv, c, E1), across<2>(m, lv, c, E2)};
+    double fs[5], u[5], w[5], un[5], wn[5];
     T ws[5];
-    int key[3];
+    load5(m, m.uold, n[0].X, u);
+    load5(m, m.uold, n[0].X2, w);
     auto pass = [&](auto dc) {
         constexpr int D = decltype(dc)::value;
         DimFlux<T> f;
-        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, k8, ok, f, ws, key[D], s_x, t);
+        auto next = [&]() {
+            if constexpr (D < 2) {
+                load5(m, m.uold, n[D + 1].X, un);
+                load5(m, m.uold, n[D + 1].X2, wn);
+            } else {
+                load5(m, a.pre, c.cC, un);
+            }
+        };
+        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n[D], u, w, k8, ok, f, ws,
+                                         s_x, t, next);
+        copy5(un, u);
+        copy5(wn, w);
         const bool par = (c.ic0 >> D) & 1;
         if constexpr (D < 2)
 #pragma unroll
@@ -636,36 +737,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
                 fs[rot<D>(i)] = i == 1 ? flip(v, par ? (int)0x80000000 : 0) : v;
             }
         } else {
-            T first[5], second[5];
-            own_terms<D>(f, par, first, second);
-#pragma unroll
-            for (int iv = 0; iv < 5; ++iv) fs[iv] = (fs[iv] + (double)first[iv]) + (double)second[iv];
+            add_own<D>(fs, f, par);
         }
     };
     pass(std::integral_constant<int, 0>{});
     pass(std::integral_constant<int, 1>{});
     pass(std::integral_constant<int, 2>{});
-    load_u(a.pre, m.ncell, c.cC, u);
+    const int key[3] = {n[0].E * 4, n[1].E * 4 + 1, n[2].E * 4 + 2};
+    ok = ok & applies_to(u);
     apply(u, fs, ws, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
-    if (!all_lanes(ok)) {
-        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, u);
+    if (__builtin_expect(!all_lanes(ok), 0)) {
+        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, u);
     }
     finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a.cpart, a.ckeys, a.courant_factor);
-}
-
-// Own terms of one dimension, signs and order as own_terms().
-template <int D, typename T> RH_DEV void put_terms(const T first[5], const T second[5], T (*s_o)[64], int t) {
-#pragma unroll
-    for (int iv = 0; iv < 5; ++iv) {
-        s_o[10 * (D - 1) + iv][t] = first[iv];
-        s_o[10 * (D - 1) + 5 + iv][t] = second[iv];
-    }
 }
 
 template <int R, bool MIXED, bool EXACT, bool SHARED>
 __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_DIMS_WAVES_F : RH_DIMS_WAVES, 8))) void k_step_dims(StepArgs a) {
     using T = typename std::conditional<MIXED, float, double>::type;
-    // Contributions of X and S per dimension, own terms of dimensions 1 and 2
+    // Contributions of X and S per dimension, own fluxes of dimensions 1 and 2
     // for the first wave, the oct across per dimension, range votes.
     __shared__ T s_x[30][64];
     __shared__ T s_o[20][64];
@@ -688,8 +778,13 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
         constexpr int D = decltype(dc)::value;
         DimFlux<T> f;
         T ws[5];
-        int kd;
-        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, k8, ok, f, ws, kd, s_x, t);
+        double u[5], w[5];
+        const Across n = across<D>(m, lv, c, oct_across<D>(lv, c));
+        load5(m, m.uold, n.X, u);
+        load5(m, m.uold, n.X2, w);
+        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n, u, w, k8, ok, f, ws, s_x, t,
+                                         [] {});
+        const int kd = n.E * 4 + D;
         const bool par = (c.ic0 >> D) & 1;
 #pragma unroll
         for (int iv = 0; iv < 5; ++iv) s_x[15 + 5 * D + iv][t] = ws[iv];
@@ -702,9 +797,11 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
             }
         } else {
             s_key[D - 1][t] = kd;
-            T first[5], second[5];
-            own_terms<D>(f, par, first, second);
-            put_terms<D>(first, second, s_o, t);
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                s_o[10 * (D - 1) + i][t] = f.Fe[i];
+                s_o[10 * (D - 1) + 5 + i][t] = f.Fi[i];
+            }
         }
         const bool bad = !all_lanes(ok);  // every lane votes
         if (t == 0) s_bad[D] = bad;
@@ -714,20 +811,28 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
     else pass(std::integral_constant<int, 2>{});
     __syncthreads();
     if (d != 0) return;
+    auto other = [&](auto dc) {
+        constexpr int D = decltype(dc)::value;
+        DimFlux<T> f;
+        key[D] = s_key[D - 1][t];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        key[1 + j] = s_key[j][t];
-#pragma unroll
-        for (int iv = 0; iv < 5; ++iv) fs[iv] = (fs[iv] + (double)s_o[10 * j + iv][t]) + (double)s_o[10 * j + 5 + iv][t];
-    }
+        for (int i = 0; i < 5; ++i) {
+            f.Fe[i] = s_o[10 * (D - 1) + i][t];
+            f.Fi[i] = s_o[10 * (D - 1) + 5 + i][t];
+        }
+        add_own<D>(fs, f, (c.ic0 >> D) & 1);
+    };
+    other(std::integral_constant<int, 1>{});
+    other(std::integral_constant<int, 2>{});
     double u[5];
     T ws2[5];
 #pragma unroll
     for (int iv = 0; iv < 5; ++iv) ws2[iv] = s_x[25 + iv][t];
-    load_u(a.pre, m.ncell, c.cC, u);
+    load5(m, a.pre, c.cC, u);
+    ok = applies_to(u) && !(s_bad[0] | s_bad[1] | s_bad[2]);
     apply(u, fs, ws2, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
-    if (s_bad[0] | s_bad[1] | s_bad[2]) {
-        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, u);
+    if (__builtin_expect(!all_lanes(ok), 0)) {
+        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, u);
     }
     finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a.cpart, a.ckeys, a.courant_factor);
 }

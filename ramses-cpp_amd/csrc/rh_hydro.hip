@@ -2259,7 +2259,7 @@ template <int R, bool MIXED, bool EXACT>
 void launch_form(int variant, const MeshDev& m, const LevelDev& lv, const GasParams& gp, const double* d_dt,
                  double dx, double inv_dx, const FusedCourant& fc, hipStream_t stream) {
     const double* pre = fc.pre_from_uold ? m.uold : m.unew;
-    if ((variant == 2 || variant == 6) && step_kernels_take(gp)) {
+    if ((variant == 2 || variant == 6) && step_kernels_take(gp, m.ncell)) {
         StepArgs a{m, lv, gp, d_dt, dx, inv_dx, pre, fc.part, fc.keys, fc.courant_factor};
         launch_step<R>(MIXED, variant == 6, a, stream);
     } else if (variant == 6) {
