@@ -3,6 +3,7 @@
 // rh_hydro.hip.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <utility>
 #include <cmath>
@@ -16,6 +17,7 @@
 #include "rh_godunov.h"
 #include "rh_guard.h"
 #include "rh_kernels.h"
+#include "rh_stage.h"
 #include "rh_tables.h"
 #include "rhydro.h"
 #include "rhydro_driver.h"
@@ -253,6 +255,16 @@ int post_call(rh_ctx* c, int what) {
     return RH_OK;
 }
 
+// Small results (time steps) to the caller, through pinned memory: a copy of
+// a few bytes into pageable memory costs as much as a launch.
+int small_to_host(rh_ctx* c, void* dst, const void* dev, size_t bytes) {
+    void* pin = bytes <= PIN_BYTES ? pinned_small(c) : nullptr;
+    RH_HIP(c, hipMemcpyAsync(pin ? pin : dst, dev, bytes, hipMemcpyDeviceToHost, c->stream));
+    RH_HIP(c, hipStreamSynchronize(c->stream));
+    if (pin) std::memcpy(dst, pin, bytes);
+    return RH_OK;
+}
+
 hipEvent_t take_event(rh_ctx* c) {
     if (!c->ev_pool.empty()) {
         hipEvent_t e = c->ev_pool.back();
@@ -333,6 +345,9 @@ void unbind(rh_ctx* c) {
     c->mesh = rh_mesh{};
 }
 
+// Octs per launch of rh_interpol_hydro (its pinned buffer is at most 4.9 MB).
+constexpr int INTERPOL_BATCH = 8192;
+
 int do_courant(rh_ctx* c, const rh::LevelDev* lv, double dx, double gamma, double cf, double* d_out,
                bool set_unew = false, const rh::AmrTimesArgs& at = rh::AmrTimesArgs{}) {
     int st = ensure_part(c, rh::courant_blocks(*lv) + 1);
@@ -345,11 +360,14 @@ int do_courant(rh_ctx* c, const rh::LevelDev* lv, double dx, double gamma, doubl
     return RH_OK;
 }
 
-int do_godunov(rh_ctx* c, const rh::LevelDev* lv, const double* d_dt, double dx, bool pre_from_uold = false) {
+// d_dt null: the time step is dt (only where launch_godunov takes it by value).
+int do_godunov(rh_ctx* c, const rh::LevelDev* lv, const double* d_dt, double dx, bool pre_from_uold = false,
+               double dt = 0.0) {
     Timed tm(c, TK_GODUNOV);
     rh::FusedCourant fc;
     const int var = variant_for(c, *lv);
     fc.pre_from_uold = pre_from_uold && var != 0;
+    fc.dt = dt;
     hipError_t e = rh::launch_godunov(mesh_dev(c), *lv, gas(c, c->p.gamma), c->p.riemann, c->p.precision, var,
                                       d_dt, dx, exact_inverse(dx), c->stream, fc);
     if (e == hipErrorNotSupported) return fail(c, RH_ERR_UNSUPPORTED, "riemann/precision combination not supported");
@@ -444,8 +462,10 @@ int rh_destroy(rh_ctx* c) {
         (void)hipSetDevice(c->p.device);
         if (c->stream) (void)hipStreamSynchronize(c->stream);
         unbind(c);
-        for (void* p : {(void*)c->d_part, (void*)c->d_dt, (void*)c->d_u1, (void*)c->d_u2})
+        for (void* p : {(void*)c->d_part, (void*)c->d_dt})
             if (p) (void)hipFree(p);
+        if (c->h_interpol) (void)hipHostFree(c->h_interpol);
+        stage_release(c);
         collect_timers(c);
         for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
         if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -587,9 +607,13 @@ int rh_godunov_fine(rh_ctx* c, int ilevel, double dt, double dx) {
         if ((st = pre_call(c))) return st;
         const rh::LevelDev* lv;
         if ((st = get_level(c, ilevel, &lv))) return st;
-        if ((st = ensure_dt(c, 1))) return st;
-        RH_HIP(c, hipMemcpyAsync(c->d_dt, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream));
-        if ((st = do_godunov(c, lv, c->d_dt, dx))) return st;
+        if (rh::takes_dt_by_value(variant_for(c, *lv), gas(c, c->p.gamma), c->mesh.ncell)) {
+            if ((st = do_godunov(c, lv, nullptr, dx, false, dt))) return st;
+        } else {
+            if ((st = ensure_dt(c, 1))) return st;
+            RH_HIP(c, hipMemcpyAsync(c->d_dt, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream));
+            if ((st = do_godunov(c, lv, c->d_dt, dx))) return st;
+        }
         RH_HIP(c, hipStreamSynchronize(c->stream));  // dt staging value is on the stack
         return post_call(c, RH_UNEW);
     });
@@ -604,11 +628,16 @@ int rh_courant(rh_ctx* c, int ilevel, double dx, double gamma, double courant_fa
         if ((st = pre_call(c))) return st;
         const rh::LevelDev* lv;
         if ((st = get_level(c, ilevel, &lv))) return st;
+        // The reduction writes the time step into pinned memory itself.
+        if (double* pin = (double*)pinned_small(c)) {
+            if ((st = do_courant(c, lv, dx, gamma, courant_factor, pin))) return st;
+            RH_HIP(c, hipStreamSynchronize(c->stream));
+            *dt_out = *pin;
+            return RH_OK;
+        }
         if ((st = ensure_dt(c, 1))) return st;
         if ((st = do_courant(c, lv, dx, gamma, courant_factor, c->d_dt))) return st;
-        RH_HIP(c, hipMemcpyAsync(dt_out, c->d_dt, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        RH_HIP(c, hipStreamSynchronize(c->stream));
-        return RH_OK;
+        return small_to_host(c, dt_out, c->d_dt, sizeof(double));
     });
 }
 
@@ -648,24 +677,33 @@ int rh_interpol_hydro(rh_ctx* c, int n_octs, const double* u1, double* u2) {
         if (n_octs < 0 || (n_octs > 0 && (!u1 || !u2))) return fail(c, RH_ERR_ARG, "bad interpol arguments");
         if (n_octs == 0) return RH_OK;
         RH_HIP(c, hipSetDevice(c->p.device));
-        if (n_octs > c->interpol_cap) {
-            if (c->d_u1) (void)hipFree(c->d_u1);
-            if (c->d_u2) (void)hipFree(c->d_u2);
-            c->d_u1 = c->d_u2 = nullptr;
+        // Of each row of 64 only the five hydro variables take part (rows keep
+        // the others as the caller passed them), so those go to pinned memory,
+        // variable by variable, which the kernel reads and writes in place.
+        const int batch = std::min(n_octs, INTERPOL_BATCH);
+        if (batch > c->interpol_cap) {
+            if (c->h_interpol) (void)hipHostFree(c->h_interpol);
+            c->h_interpol = nullptr;
             c->interpol_cap = 0;
-            RH_HIP(c, hipMalloc(&c->d_u1, (size_t)n_octs * 7 * 64 * sizeof(double)));
-            RH_HIP(c, hipMalloc(&c->d_u2, (size_t)n_octs * 8 * 64 * sizeof(double)));
-            c->interpol_cap = n_octs;
+            const int cap = std::min(INTERPOL_BATCH, std::max(64, batch + batch / 4));
+            RH_HIP(c, hipHostMalloc((void**)&c->h_interpol, (size_t)cap * 75 * sizeof(double), hipHostMallocDefault));
+            c->interpol_cap = cap;
         }
-        RH_HIP(c, hipMemcpyAsync(c->d_u1, u1, (size_t)n_octs * 7 * 64 * sizeof(double), hipMemcpyHostToDevice,
-                                 c->stream));
-        // Rows beyond nvar are returned unchanged from what the caller passed.
-        RH_HIP(c, hipMemcpyAsync(c->d_u2, u2, (size_t)n_octs * 8 * 64 * sizeof(double), hipMemcpyHostToDevice,
-                                 c->stream));
-        RH_HIP(c, rh::launch_interpol(n_octs, c->d_u1, c->d_u2, gas(c, c->p.gamma), c->p.interpol_var, c->stream));
-        RH_HIP(c, hipMemcpyAsync(u2, c->d_u2, (size_t)n_octs * 8 * 64 * sizeof(double), hipMemcpyDeviceToHost,
-                                 c->stream));
-        RH_HIP(c, hipStreamSynchronize(c->stream));
+        for (int o0 = 0; o0 < n_octs; o0 += batch) {
+            const int n = std::min(batch, n_octs - o0);
+            double* in = c->h_interpol;
+            double* out = in + (size_t)35 * n;
+            for (int o = 0; o < n; ++o)
+                for (int i = 0; i < 7; ++i)
+                    for (int iv = 0; iv < 5; ++iv)
+                        in[(size_t)(i * 5 + iv) * n + o] = u1[((size_t)(o0 + o) * 7 + i) * 64 + iv];
+            RH_HIP(c, rh::launch_interpol(n, in, out, gas(c, c->p.gamma), c->p.interpol_var, c->stream));
+            RH_HIP(c, hipStreamSynchronize(c->stream));
+            for (int o = 0; o < n; ++o)
+                for (int i = 0; i < 8; ++i)
+                    for (int iv = 0; iv < 5; ++iv)
+                        u2[((size_t)(o0 + o) * 8 + i) * 64 + iv] = out[(size_t)(i * 5 + iv) * n + o];
+        }
         return RH_OK;
     });
 }
@@ -782,10 +820,11 @@ int rh_run_uniform(rh_ctx* c, int ilevel, double dx, double courant_factor, int 
                 tm.done();
             }
         }
-        if (dt_out && nsteps > 0)
-            RH_HIP(c, hipMemcpyAsync(dt_out, c->d_dt, (size_t)nsteps * sizeof(double), hipMemcpyDeviceToHost,
-                                     c->stream));
-        RH_HIP(c, hipStreamSynchronize(c->stream));
+        if (dt_out && nsteps > 0) {
+            if ((st = small_to_host(c, dt_out, c->d_dt, (size_t)nsteps * sizeof(double)))) return st;
+        } else {
+            RH_HIP(c, hipStreamSynchronize(c->stream));
+        }
         return post_call(c, RH_UOLD | RH_UNEW);
     });
 }

@@ -84,9 +84,11 @@ struct rh_ctx {
     int npart = 0;
     double* d_dt = nullptr;
     int ndt = 0;
-    double* d_u1 = nullptr;
-    double* d_u2 = nullptr;
+    // Pinned operands and results of rh_interpol_hydro (75 doubles per oct).
+    double* h_interpol = nullptr;
     int interpol_cap = 0;
+    // Pinned memory for small results (pinned_small).
+    void* h_pin = nullptr;
     // Godunov kernel variant (rh_set_kernel_variant, rh_autotune); -1: the
     // default, chosen per level by variant_for.
     int variant = -1;
@@ -138,6 +140,8 @@ int ensure_dt(rh_ctx* c, int n);
 // Level tables of ilevel for the bound mesh, rebuilt when the epoch moved.
 int get_level(rh_ctx* c, int ilevel, const rh::LevelDev** out);
 void collect_timers(rh_ctx* c);
+// Copies a small device result to the caller and waits for the stream.
+int small_to_host(rh_ctx* c, void* dst, const void* dev, size_t bytes);
 // A single mesh is bound (not an ensemble); else an error on c.
 int check_bound(rh_ctx* c);
 // Host-coherent mode: uploads the host state (and f) before a call.

@@ -390,10 +390,11 @@ int rh_run_ensemble(rh_ctx* c, const int* levels, const double* dx, double coura
                 tm.done();
             }
         }
-        if (dt_out && nsteps > 0)
-            RH_HIP(c, hipMemcpyAsync(dt_out, c->d_dt, (size_t)nsteps * nbox * sizeof(double), hipMemcpyDeviceToHost,
-                                     c->stream));
-        RH_HIP(c, hipStreamSynchronize(c->stream));
+        if (dt_out && nsteps > 0) {
+            if ((st = small_to_host(c, dt_out, c->d_dt, (size_t)nsteps * nbox * sizeof(double)))) return st;
+        } else {
+            RH_HIP(c, hipStreamSynchronize(c->stream));
+        }
         if (c->mode == RH_HOST_COHERENT) return ens_download_state(c, RH_UOLD | RH_UNEW);
         return RH_OK;
     });

@@ -14,7 +14,8 @@ struct StepArgs {
     MeshDev m;
     LevelDev lv;
     GasParams gp;
-    const double* d_dt;
+    const double* d_dt;  // null: the time step is dt (a single mesh)
+    double dt;
     double dx, inv_dx;
     const double* pre;
     double* cpart;

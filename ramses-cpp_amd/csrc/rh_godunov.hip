@@ -218,7 +218,8 @@ RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, T (*w)[64], 
     const GasParams& gp = a.gp;
     const Rows<T> W{w, t};
     double dt, dx = a.dx, inv_dx = a.inv_dx;
-    step_of(lv, p, a.d_dt, dt, dx, inv_dx);
+    if (a.d_dt) step_of(lv, p, a.d_dt, dt, dx, inv_dx);
+    else dt = a.dt;
     const double dtdx = dt / dx;
     double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, F[5];
     load_u(a.pre, m.ncell, cC, u);
@@ -576,7 +577,7 @@ RH_DEV bool constants(const StepArgs& a, int p, double& dt, double& dx, Consts<T
         dx = a.lv.box_len[box];
         inv_dx = a.lv.box_len[a.lv.nbox + box];
     } else {
-        dt = *a.d_dt;
+        dt = a.d_dt ? *a.d_dt : a.dt;
     }
     dt = uniform(dt);
     dx = uniform(dx);

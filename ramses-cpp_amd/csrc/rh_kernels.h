@@ -122,10 +122,13 @@ struct FusedCourant {
     double* part = nullptr;
     unsigned long long* keys = nullptr;
     double courant_factor = 0.0;
+    double dt = 0.0;  // the time step when d_dt is null (takes_dt_by_value)
 };
 hipError_t launch_godunov(const MeshDev& m, const LevelDev& lv, const GasParams& gp, int riemann, int precision,
                           int variant, const double* d_dt, double dx, double inv_dx, hipStream_t stream,
                           const FusedCourant& fc = FusedCourant{});
+// Whether launch_godunov takes the time step by value (d_dt null) there.
+bool takes_dt_by_value(int variant, const GasParams& gp, int ncell);
 int godunov_blocks(const LevelDev& lv, int variant);
 // Minimum of part[0..nparts) and dt_init into *d_dt (the Courant step); part is
 // overwritten when it is long.
@@ -170,7 +173,10 @@ constexpr int AMR_T_SIZE = 3 * AMR_T_LEVELS + 2;
 hipError_t launch_flag_bits(const MeshDev& m, const LevelDev& lv, const int* d_nbor, double ed, double ep,
                             double ev, double gamma, int nexpand, unsigned char* d_a, unsigned char* d_b,
                             unsigned char** d_result, hipStream_t stream);
-hipError_t launch_interpol(int n_octs, const double* d_u1, double* d_u2, const GasParams& gp, int interpol_var,
+// Prolongation of n octs: u1[(i*5+iv)*n + o] variable iv of row i (the cell,
+// then its six neighbours) of oct o, u2[(i*5+iv)*n + o] of child i; both may
+// be pinned host memory.
+hipError_t launch_interpol(int n_octs, const double* u1, double* u2, const GasParams& gp, int interpol_var,
                            hipStream_t stream);
 // Snapshot hydro records of one level list (n grids, d_grids in list order)
 // as 32-bit words, pack_hydro_words(n, nbnd) of them, into d_out.
