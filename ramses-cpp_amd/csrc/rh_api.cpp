@@ -17,6 +17,7 @@
 #include "rh_godunov.h"
 #include "rh_guard.h"
 #include "rh_kernels.h"
+#include "rh_pool.h"
 #include "rh_stage.h"
 #include "rh_tables.h"
 #include "rhydro.h"
@@ -213,19 +214,18 @@ size_t state_bytes(const rh_ctx* c) { return (size_t)c->mesh.nvar * c->mesh.ncel
 
 int upload_state(rh_ctx* c, int what) {
     if (c->ens) return ens_upload_state(c, what);
-    if (what & RH_UOLD)
-        RH_HIP(c, hipMemcpyAsync(c->d_uold, c->mesh.uold, state_bytes(c), hipMemcpyHostToDevice, c->stream));
-    if (what & RH_UNEW)
-        RH_HIP(c, hipMemcpyAsync(c->d_unew, c->mesh.unew, state_bytes(c), hipMemcpyHostToDevice, c->stream));
-    return RH_OK;
+    int st = RH_OK;
+    if (what & RH_UOLD) st = stage_to_device(c, {{c->mesh.uold, state_bytes(c)}}, c->d_uold);
+    if (st == RH_OK && (what & RH_UNEW)) st = stage_to_device(c, {{c->mesh.unew, state_bytes(c)}}, c->d_unew);
+    return st;
 }
 
 int download_state(rh_ctx* c, int what) {
     if (c->ens) return ens_download_state(c, what);
-    if (what & RH_UOLD)
-        RH_HIP(c, hipMemcpyAsync(c->mesh.uold, c->d_uold, state_bytes(c), hipMemcpyDeviceToHost, c->stream));
-    if (what & RH_UNEW)
-        RH_HIP(c, hipMemcpyAsync(c->mesh.unew, c->d_unew, state_bytes(c), hipMemcpyDeviceToHost, c->stream));
+    int st = RH_OK;
+    if (what & RH_UOLD) st = stage_to_host(c, {{c->mesh.uold, state_bytes(c)}}, c->d_uold);
+    if (st == RH_OK && (what & RH_UNEW)) st = stage_to_host(c, {{c->mesh.unew, state_bytes(c)}}, c->d_unew);
+    if (st) return st;
     RH_HIP(c, hipStreamSynchronize(c->stream));
     return RH_OK;
 }
@@ -245,8 +245,7 @@ int pre_call(rh_ctx* c) {
     if (st) return st;
     // The host's gravity solver may have updated f since the last call.
     if (c->d_f && c->mesh.f)
-        RH_HIP(c, hipMemcpyAsync(c->d_f, c->mesh.f, (size_t)3 * c->mesh.ncell * sizeof(double),
-                                 hipMemcpyHostToDevice, c->stream));
+        return stage_to_device(c, {{const_cast<double*>(c->mesh.f), (size_t)3 * c->mesh.ncell * sizeof(double)}}, c->d_f);
     return RH_OK;
 }
 
@@ -517,7 +516,7 @@ int rh_bind(rh_ctx* c, const rh_mesh* m, int mode) {
                 RH_HIP(c, hipMalloc(&c->d_f, nf * sizeof(double)));
                 c->f_cap = nf;
             }
-            RH_HIP(c, hipMemcpyAsync(c->d_f, m->f, nf * sizeof(double), hipMemcpyHostToDevice, c->stream));
+            if ((st = stage_to_device(c, {{const_cast<double*>(m->f), nf * sizeof(double)}}, c->d_f))) return st;
         } else if (c->d_f) {
             (void)hipFree(c->d_f);
             c->d_f = nullptr;
