@@ -45,6 +45,7 @@
 #include "rhydro_driver.h"
 #include "rhydro_snapshot.h"
 #include "rh_snapshot.h"
+#include "rh_stage.h"
 
 struct rh_amr {
     rh_ctx* ctx = nullptr;
@@ -80,6 +81,10 @@ struct rh_amr {
     unsigned char* d_flags = nullptr;  // 8*ngridmax bytes: two flag buffers of flag_fine
     unsigned char* h_flags = nullptr;  // ngridmax bytes of pinned host memory: a list's flags
     double* d_times = nullptr;  // rh::AMR_T_SIZE doubles
+    // Operands of apply_all, while the run is being set up.
+    double* d_init = nullptr;
+    size_t init_cap = 0;
+    std::vector<double> init_host;
     // Each level list's grids in list order, and the edit count of the list
     // they were read at (list_version is bumped by every edit of the list).
     std::vector<std::vector<int>> list_cache;
@@ -868,55 +873,96 @@ int restrict_fine(rh_amr* a, int il) {
     return RH_OK;
 }
 
-// Initializer.cpp:19-157 (apply_all) computed on the host for every coarse
-// and listed cell, then uploaded.  Cells that no region covers keep their
-// state, so the current device state is the starting point.
+// Initializer.cpp:19-157 (apply_all) for every coarse and listed cell, on the
+// device: the host lays out the octs' centres in list order (and the shear
+// layer's velocities) and the regions' states.
 int apply_all(rh_amr* a) {
     const bool kh = a->ap.ic_kind == 1;
-    auto set = [&](int idc, double d, double u, double v, double w, double p) {
-        auto U = [&](int iv) -> double& { return a->uold[(size_t)(iv - 1) * a->ncell + idc - 1]; };
-        U(1) = d;
-        U(2) = d * u;
-        U(3) = d * v;
-        U(4) = d * w;
+    const int nreg = (int)a->reg_type.size(), nc = a->ncoarse;
+    // Each level's device list by value: get_level may move the tables of the
+    // others.
+    std::vector<const int*> grid(a->nlevelmax + 1, nullptr);
+    std::vector<int> num(a->nlevelmax + 1, 0);
+    num[0] = nc;
+    size_t cells = nc;
+    for (int il = 1; il <= a->nlevelmax; ++il) {
+        if (count(a, il) == 0) continue;
+        const rh::LevelDev* lv;
+        RH_ACHK(get_level(a->ctx, il, &lv));
+        if (lv->noct != count(a, il)) return afail(a, RH_ERR_HOST, "level list and level tables disagree");
+        grid[il] = lv->grid;
+        num[il] = lv->noct;
+        cells += lv->noct;
+    }
+    // Regions, then per list three coordinates and two velocities.
+    std::vector<double>& h = a->init_host;
+    const size_t need = (size_t)12 * nreg + 5 * cells;
+    if (need > h.size()) h.resize(need);
+    if (need > a->init_cap) {
+        if (a->d_init) (void)hipFree(a->d_init);
+        a->d_init = nullptr;
+        a->init_cap = 0;
+        RH_AHIP(a, hipMalloc(&a->d_init, need * sizeof(double)));
+        a->init_cap = need;
+    }
+    for (int r = 0; r < nreg; ++r) {
+        const bool box = a->reg_type[r] == 0;
+        const double d = a->reg[6][r], u = a->reg[7][r], v = a->reg[8][r], w = a->reg[9][r], p = a->reg[10][r];
         double v2 = u * u;
         v2 += v * v;
         v2 += w * w;
-        double e_kin = 0.5 * d * v2;
-        double e_int = p / (a->gamma - 1.0);
-        double e_nonthermal = 0.0;
-        U(5) = e_kin + e_int + e_nonthermal;
-    };
-    auto apply = [&](int idc) {
-        double xc[3];
-        cell_center(a, idc, xc);
-        const double x = xc[0], y = xc[1], z = xc[2];
-        if (kh) {
-            const double pi = 3.14159265358979323846;
-            const bool in = std::abs(y - 0.5) < 0.25;
-            set(idc, in ? 2.0 : 1.0, in ? 0.5 : -0.5, a->ap.kh_amp * std::sin(4.0 * pi * x), 0.0, 2.5);
-            return;
+        const double e_kin = 0.5 * d * v2, e_int = p / (a->gamma - 1.0), e_nonthermal = 0.0;
+        const double row[12] = {box ? 0.0 : 1.0, a->reg[0][r], a->reg[1][r], a->reg[2][r],
+                                box ? 0.5 * a->reg[3][r] : std::pow(a->reg[3][r], 2), 0.5 * a->reg[4][r],
+                                0.5 * a->reg[5][r], d, d * u, d * v, d * w, e_kin + e_int + e_nonthermal};
+        for (int k = 0; k < 12; ++k) h[(size_t)k * nreg + r] = row[k];
+    }
+    const double pi = 3.14159265358979323846;
+    auto layer = [&](double x) { return a->ap.kh_amp * std::sin(4.0 * pi * x); };
+    size_t at = (size_t)12 * nreg;
+    std::vector<size_t> begin(a->nlevelmax + 1, 0);
+    // The coarse octs make up list 2, so the cells of list il are
+    // boxlen / (nx * 2^(il-1)) wide.
+    auto width = [&](int il) { return a->boxlen / (double)(a->nx * (1 << (il - 1))); };
+    for (int il = 0; il <= a->nlevelmax; ++il) {
+        const int n = num[il];
+        if (n == 0) continue;
+        double* q = h.data() + at;
+        begin[il] = at;
+        at += (size_t)5 * n;
+        if (il == 0) {
+            for (int i = 0; i < nc; ++i) {
+                double xc[3];
+                cell_center(a, i + 1, xc);
+                for (int d = 0; d < 3; ++d) q[(size_t)d * n + i] = xc[d];
+                if (kh) q[(size_t)3 * n + i] = layer(xc[0]);
+            }
+            continue;
         }
-        for (size_t r = 0; r < a->reg_type.size(); ++r) {
-            const double xr = a->reg[0][r], yr = a->reg[1][r], zr = a->reg[2][r];
-            bool in;
-            if (a->reg_type[r] == 0)
-                in = std::abs(x - xr) < 0.5 * a->reg[3][r] && std::abs(y - yr) < 0.5 * a->reg[4][r] &&
-                     std::abs(z - zr) < 0.5 * a->reg[5][r];
-            else
-                in = std::pow(x - xr, 2) + std::pow(y - yr, 2) + std::pow(z - zr, 2) < std::pow(a->reg[3][r], 2);
-            if (in) set(idc, a->reg[6][r], a->reg[7][r], a->reg[8][r], a->reg[9][r], a->reg[10][r]);
-        }
-    };
-    RH_AHIP(a, hipMemcpyAsync(a->uold.data(), a->ctx->d_uold, a->uold.size() * sizeof(double),
-                              hipMemcpyDeviceToHost, a->ctx->stream));
-    RH_AHIP(a, hipStreamSynchronize(a->ctx->stream));
-    for (int i = 1; i <= a->ncoarse; ++i) apply(i);
-    for (int il = 1; il <= a->nlevelmax; ++il)
-        for (int ig = a->headl[il]; ig > 0; ig = a->next[ig - 1])
-            for (int ic = 1; ic <= 8; ++ic) apply(cell(a, ig, ic));
-    RH_AHIP(a, hipMemcpyAsync(a->ctx->d_uold, a->uold.data(), a->uold.size() * sizeof(double),
-                              hipMemcpyHostToDevice, a->ctx->stream));
+        const std::vector<int>& grids = list_grids(a, il);
+        if ((int)grids.size() != n) return afail(a, RH_ERR_HOST, "level list and level tables disagree");
+        const double dx = width(il), scale = a->boxlen / (double)a->nx;
+        parallel_for(n, [&](int k) {
+            for (int d = 0; d < 3; ++d) q[(size_t)d * n + k] = a->xg[(size_t)d * a->ngridmax + grids[k] - 1];
+            if (kh)
+                for (int i = 0; i < 2; ++i) q[(size_t)(3 + i) * n + k] = layer(q[k] * scale + ((double)i - 0.5) * dx);
+        });
+    }
+    RH_ACHK(stage_to_device(a->ctx, {{h.data(), at * sizeof(double)}}, a->d_init));
+    for (int il = 0; il <= a->nlevelmax; ++il) {
+        if (num[il] == 0) continue;
+        rh::InitialArgs ia{};
+        ia.grid = grid[il];
+        ia.n = num[il];
+        ia.pos = a->d_init + begin[il];
+        ia.scale = a->boxlen / (double)a->nx;
+        ia.dx = il > 0 ? width(il) : 0.0;
+        if (kh) ia.vel = ia.pos + (size_t)3 * ia.n;
+        ia.e_int = 2.5 / (a->gamma - 1.0);
+        ia.reg = a->d_init;
+        ia.nreg = nreg;
+        RH_AHIP(a, rh::launch_initial(mesh_dev(a->ctx), ia, a->ctx->stream));
+    }
     RH_AHIP(a, hipStreamSynchronize(a->ctx->stream));
     return RH_OK;
 }
@@ -949,7 +995,12 @@ int initialize(rh_amr* a) {
         if (count(a, il_ref) == 0) break;
     }
     a->nstep = 0;
-    return legacy_init_flow(a);
+    RH_ACHK(legacy_init_flow(a));
+    (void)hipFree(a->d_init);
+    a->d_init = nullptr;
+    a->init_cap = 0;
+    std::vector<double>().swap(a->init_host);
+    return RH_OK;
 }
 
 // Simulation.cpp:522-635
@@ -1038,7 +1089,8 @@ void destroy(rh_amr* a) {
     if (a->ctx) {
         (void)hipSetDevice(a->hp.device);
         (void)hipStreamSynchronize(a->ctx->stream);
-        for (void* p : {(void*)a->d_father, (void*)a->d_nbor, (void*)a->d_cells, (void*)a->d_flags, (void*)a->d_times})
+        for (void* p : {(void*)a->d_father, (void*)a->d_nbor, (void*)a->d_cells, (void*)a->d_flags, (void*)a->d_times,
+                        (void*)a->d_init})
             if (p) (void)hipFree(p);
         if (a->h_flags) (void)hipHostFree(a->h_flags);
         if (a->h_cells) (void)hipHostFree(a->h_cells);

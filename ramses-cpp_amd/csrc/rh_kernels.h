@@ -154,6 +154,25 @@ hipError_t launch_restrict(const MeshDev& m, const LevelDev& fine, const int* d_
 // set_uold of lv and the restriction of fine (the next finer level) into it, one launch.
 hipError_t launch_set_uold_restrict(const MeshDev& m, const LevelDev& lv, const LevelDev& fine, const int* d_father,
                                     hipStream_t stream);
+// Initial conditions of n octs (grid: their list) or of the n coarse cells
+// (grid null) into uold.
+struct InitialArgs {
+    const int* grid;
+    int n;
+    const double* pos;  // [3][n]: the octs' centres in units of scale, or the coarse cells' centres
+    double scale, dx;   // of an oct's cells
+    // The shear layer, or null: transverse velocity of each oct's cells,
+    // [2][n] by the cell's side in x ([n] for coarse cells), and the thermal
+    // energy.
+    const double* vel;
+    double e_int;
+    // Otherwise regions, [12][nreg]: 0 for a box, else a sphere; centre; a
+    // box's half lengths or a sphere's squared radius; conserved state.  The
+    // last one that holds a cell's centre counts.
+    const double* reg;
+    int nreg;
+};
+hipError_t launch_initial(const MeshDev& m, const InitialArgs& a, hipStream_t stream);
 // Adaptive run's time-step table on the device (doubles): dtnew, dtold and
 // the dt each level's last step used, AMR_T_LEVELS entries each, then the
 // time t and the latest Courant minimum.
