@@ -201,6 +201,16 @@ int ensure_part(rh_ctx* c, int n) {
     return RH_OK;
 }
 
+int ensure_keys(rh_ctx* c, int n) {
+    if (n <= c->nkeys) return RH_OK;
+    if (c->d_keys) (void)hipFree(c->d_keys);
+    c->d_keys = nullptr;
+    c->nkeys = 0;
+    RH_HIP(c, hipMalloc(&c->d_keys, (size_t)n * sizeof(unsigned long long)));
+    c->nkeys = n;
+    return RH_OK;
+}
+
 int ensure_dt(rh_ctx* c, int n) {
     if (n <= c->ndt) return RH_OK;
     if (c->d_dt) (void)hipFree(c->d_dt);
@@ -343,6 +353,13 @@ void unbind(rh_ctx* c) {
     c->bound = false;
     c->mesh = rh_mesh{};
 }
+
+// Levels up to this many octs hand the Courant minimum from step to step
+// through slots: a launch less per step, for an atomic per 8 octs and one more
+// operand to wait for.  Per step (HLLC, FP64), reduced by a launch of its own
+// and through slots: 16^3 10.0 and 8.3 us, 32^3 12.6 and 11.0, 64^3 35.4 and
+// 33.5, 128^3 201 and 200.5, 256^3 1,706 and 1,715.
+constexpr int SLOTS_MAX_OCTS = 1 << 17;
 
 // Octs per launch of rh_interpol_hydro (its pinned buffer is at most 4.9 MB).
 constexpr int INTERPOL_BATCH = 8192;
@@ -752,26 +769,38 @@ int rh_run_uniform(rh_ctx* c, int ilevel, double dx, double courant_factor, int 
             if ((st = ensure_part(c, std::max(nb, rh::courant_blocks(*lv)) + 1))) return st;
             const rh::GasParams gp = gas(c, c->p.gamma);
             const double inv_dx = exact_inverse(dx), dt_init = c->p.boxlen / 1e-10;
+            // Three sets of slots: the one a step reads, the one it fills and
+            // the one it clears for the step after.
+            const int nset = rh::COURANT_SLOTS * rh::COURANT_STRIDE;
+            const bool slots = rh::takes_dt_by_value(var, gp, c->mesh.ncell) && lv->noct <= SLOTS_MAX_OCTS;
+            if (slots && (st = ensure_keys(c, 3 * nset))) return st;
             auto issue = [&]() -> int {
                 int s2;
                 rh::MeshDev mk = m;
+                if (slots) RH_HIP(c, rh::launch_fill_keys(c->d_keys, 3 * nset, dt_init, c->stream));
                 for (int k = 0; k < nsteps; ++k) {
                     if (k == 0 && (s2 = do_courant(c, lv, dx, c->p.gamma, courant_factor, c->d_dt))) return s2;
                     const bool next = k + 1 < nsteps;
                     rh::FusedCourant fc;
                     fc.pre_from_uold = true;
-                    fc.part = next ? c->d_part : nullptr;
+                    fc.part = next && !slots ? c->d_part : nullptr;
                     fc.courant_factor = courant_factor;
+                    if (slots) {
+                        auto set = [&](int i) { return c->d_keys + (size_t)(i % 3) * nset; };
+                        fc.slots = {k ? set(k) : nullptr, next ? set(k + 1) : nullptr, next ? set(k + 2) : nullptr,
+                                    c->d_dt + k, dt_init};
+                    }
                     {
                         Timed tm(c, TK_GODUNOV);
                         hipError_t e = rh::launch_godunov(mk, *lv, gp, c->p.riemann, c->p.precision, var,
-                                                          c->d_dt + k, dx, inv_dx, c->stream, fc);
+                                                          slots && k ? nullptr : c->d_dt + k, dx, inv_dx, c->stream,
+                                                          fc);
                         if (e == hipErrorNotSupported)
                             return fail(c, RH_ERR_UNSUPPORTED, "riemann/precision combination not supported");
                         if (e != hipSuccess) return hip_fail(c, e, "godunov launch");
                         tm.done();
                     }
-                    if (next) {
+                    if (next && !slots) {
                         Timed tm(c, TK_COURANT);
                         RH_HIP(c, rh::launch_courant_final(c->d_part, nb, dt_init, c->d_dt + k + 1, c->stream));
                         tm.done();
@@ -790,7 +819,7 @@ int rh_run_uniform(rh_ctx* c, int ilevel, double dx, double courant_factor, int 
             key_add(key, m);
             key_add(key, gp);
             key.add(c->p.riemann).add(c->p.precision).add(var).add(dx).add(inv_dx).add(courant_factor);
-            key.add(dt_init).add(nsteps).add(nb).add(c->d_dt).add(c->d_part).add(c->npart);
+            key.add(dt_init).add(nsteps).add(nb).add(c->d_dt).add(c->d_part).add(c->npart).add(slots).add(c->d_keys);
             if ((st = run_graph(c, c->g_uniform, key, issue))) return st;
         }
         // Otherwise step k is courant -> set_unew -> godunov_fine -> set_uold.

@@ -276,13 +276,7 @@ int rh_run_ensemble(rh_ctx* c, const int* levels, const double* dx, double coura
         const rh::LevelDev& lv = c->ens_level.dev;
         const int nk = nbox * (nsteps > 0 ? nsteps : 1);
         if ((st = ensure_dt(c, nk))) return st;
-        if (nk > c->nkeys) {
-            if (c->d_keys) (void)hipFree(c->d_keys);
-            c->d_keys = nullptr;
-            c->nkeys = 0;
-            RH_HIP(c, hipMalloc(&c->d_keys, (size_t)nk * sizeof(unsigned long long)));
-            c->nkeys = nk;
-        }
+        if ((st = ensure_keys(c, nk))) return st;
         const rh::MeshDev m = mesh_dev(c);
         const rh::GasParams gp = gas(c, c->p.gamma);
         const double dt_init = c->p.boxlen / 1e-10;

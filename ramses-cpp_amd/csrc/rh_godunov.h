@@ -8,19 +8,20 @@ namespace rh {
 // Arguments of one update launch.  dx, inv_dx: the level's cell width and its
 // exact reciprocal or 0 (an ensemble reads both per box; inv_dx != 0 when
 // every box has one); pre: the buffer the cells' state before the update is
-// read from; cpart / ckeys: where the next step's Courant candidates go, or
-// null (launch_godunov's FusedCourant).
+// read from; cpart / ckeys / slots: where the next step's Courant candidates
+// go, or null (launch_godunov's FusedCourant).
 struct StepArgs {
     MeshDev m;
     LevelDev lv;
     GasParams gp;
-    const double* d_dt;  // null: the time step is dt (a single mesh)
+    const double* d_dt;  // null: the time step is the slots' or dt (a single mesh)
     double dt;
     double dx, inv_dx;
     const double* pre;
     double* cpart;
     unsigned long long* ckeys;
     double courant_factor;
+    CourantSlots slots;
 };
 
 // Whether the update runs in these kernels for a configuration: their slope

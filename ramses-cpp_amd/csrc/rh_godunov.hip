@@ -211,6 +211,14 @@ RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& 
     }
 }
 
+// The time step in a launch's slots, for the general path.
+RH_DEV double slots_dt(const unsigned long long* in) {
+    unsigned long long k = in[0];
+#pragma unroll 1
+    for (int i = 1; i < COURANT_SLOTS; ++i) k = min(k, in[i * COURANT_STRIDE]);
+    return key_dt(k);
+}
+
 template <int R, bool MIXED, typename T>
 RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, T (*w)[64], int t, double u[5]) {
     const MeshDev& m = a.m;
@@ -219,6 +227,7 @@ RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, T (*w)[64], 
     const Rows<T> W{w, t};
     double dt, dx = a.dx, inv_dx = a.inv_dx;
     if (a.d_dt) step_of(lv, p, a.d_dt, dt, dx, inv_dx);
+    else if (a.slots.in) dt = slots_dt(a.slots.in);
     else dt = a.dt;
     const double dtdx = dt / dx;
     double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, F[5];
@@ -578,6 +587,17 @@ RH_DEV bool constants(const StepArgs& a, int p, double& dt, double& dx, Consts<T
         inv_dx = a.lv.box_len[a.lv.nbox + box];
     } else {
         dt = a.d_dt ? *a.d_dt : a.dt;
+        if (a.slots.in) {
+            unsigned long long key = a.slots.in[(threadIdx.x & (COURANT_SLOTS - 1)) * COURANT_STRIDE];
+#pragma unroll
+            for (int off = COURANT_SLOTS / 2; off > 0; off >>= 1) key = min(key, (unsigned long long)__shfl_xor(key, off, 64));
+            dt = key_dt(key);
+        }
+        if (blockIdx.x == 0) {
+            if (a.slots.in && threadIdx.x == 0) *a.slots.dt_out = dt;
+            if (a.slots.clear && threadIdx.x < COURANT_SLOTS)
+                a.slots.clear[threadIdx.x * COURANT_STRIDE] = dt_key(a.slots.dt_init);
+        }
     }
     dt = uniform(dt);
     dx = uniform(dx);
@@ -652,9 +672,12 @@ RH_DEV void apply(double u[5], const double fs[5], const T ws2[5], const T (*wx)
 // operation rounding monotonically, so the wave takes the largest sum and
 // does the divisions once.
 RH_DEV void finish(const MeshDev& m, const LevelDev& lv, const GasParams& gp, const double u[5], bool leaf, int cC, int p,
-                   int pfirst, int t, double dx, double* cpart, unsigned long long* ckeys, double courant_factor) {
+                   int pfirst, int t, double dx, const StepArgs& a) {
+    double* const cpart = a.cpart;
+    unsigned long long *const ckeys = a.ckeys, *const slots = a.slots.out;
+    const double courant_factor = a.courant_factor;
     if (leaf) store5(m, m.unew, cC, u);
-    if (!cpart && !ckeys) return;
+    if (!cpart && !ckeys && !slots) return;
     const double s1 = ssqrt(1.0 + 2.0 * courant_factor * 1e-4) - 1.0;
     const bool one_box = !ckeys || lv.obox[pfirst] == lv.obox[min(pfirst + 8, lv.noct) - 1];
     double cand = __builtin_inf();
@@ -670,6 +693,8 @@ RH_DEV void finish(const MeshDev& m, const LevelDev& lv, const GasParams& gp, co
     }
     if (cpart) {
         if (t == 0) cpart[blockIdx.x] = cand;
+    } else if (slots) {
+        if (t == 0) atomicMin(&slots[(blockIdx.x & (COURANT_SLOTS - 1)) * COURANT_STRIDE], dt_key(cand));
     } else if (one_box) {
         if (t == 0) atomicMin(&ckeys[lv.obox[pfirst]], dt_key(cand));
     } else if (cand != __builtin_inf()) {
@@ -678,15 +703,18 @@ RH_DEV void finish(const MeshDev& m, const LevelDev& lv, const GasParams& gp, co
 }
 
 // This wave's cells: 8 octs of the list, lanes past its end on the last oct.
+// Their states are loaded before the time step is taken from the slots, so
+// that the two waits overlap.
 template <typename T>
-RH_DEV void load_cell(const MeshDev& m, const LevelDev& lv, int praw, int t, const Consts<T>& k, Cell<T>& c, bool& ok) {
+RH_DEV void find_cell(const MeshDev& m, const LevelDev& lv, int praw, int t, Cell<T>& c, double u[5]) {
     c.ic0 = t & 7;
     c.p = min(praw, lv.noct - 1);
     c.lm = at(lv.leaf, c.p);
     c.leaf = praw < lv.noct && ((c.lm >> c.ic0) & 1);
     c.cC = cell_id(m, at(lv.grid, c.p), c.ic0);
-    double u[5];
     load5(m, m.uold, c.cC, u);
+}
+template <typename T> RH_DEV void take_cell(const double u[5], const Consts<T>& k, Cell<T>& c, bool& ok) {
     fast::prim(u, c.q, c.y, k, ok);
     c.c2 = fast::trace_c2(c.q[0], c.q[4], c.y, k);
 }
@@ -702,12 +730,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
     double dt, dx;
     Consts<T> k;
     Cell<T> c;
-    bool ok = constants(a, min(praw, lv.noct - 1), dt, dx, k);
-    load_cell(m, lv, praw, t, k, c, ok);
+    double u[5];
+    find_cell(m, lv, praw, t, c, u);
+    bool ok = constants(a, c.p, dt, dx, k);
+    take_cell(u, k, c, ok);
     const double dtdx = uniform(dt / dx), k8 = uniform(dtdx * 0.125);
     const int E0 = oct_across<0>(lv, c), E1 = oct_across<1>(lv, c), E2 = oct_across<2>(lv, c);
     const Across n[3] = {across<0>(m, lv, c, E0), across<1>(m, lv, c, E1), across<2>(m, lv, c, E2)};
-    double fs[5], u[5], w[5], un[5], wn[5];
+    double fs[5], w[5], un[5], wn[5];
     T ws[5];
     load5(m, m.uold, n[0].X, u);
     load5(m, m.uold, n[0].X2, w);
@@ -750,7 +780,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
     if (__builtin_expect(!all_lanes(ok), 0)) {
         if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, u);
     }
-    finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a.cpart, a.ckeys, a.courant_factor);
+    finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a);
 }
 
 template <int R, bool MIXED, bool EXACT, bool SHARED>
@@ -770,8 +800,10 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
     double dt, dx;
     Consts<T> k;
     Cell<T> c;
-    bool ok = constants(a, min(praw, lv.noct - 1), dt, dx, k);
-    load_cell(m, lv, praw, t, k, c, ok);
+    double u[5];
+    find_cell(m, lv, praw, t, c, u);
+    bool ok = constants(a, c.p, dt, dx, k);
+    take_cell(u, k, c, ok);
     const double dtdx = uniform(dt / dx), k8 = uniform(dtdx * 0.125);
     double fs[5];
     int key[3];
@@ -779,11 +811,11 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
         constexpr int D = decltype(dc)::value;
         DimFlux<T> f;
         T ws[5];
-        double u[5], w[5];
+        double x[5], w[5];
         const Across n = across<D>(m, lv, c, oct_across<D>(lv, c));
-        load5(m, m.uold, n.X, u);
+        load5(m, m.uold, n.X, x);
         load5(m, m.uold, n.X2, w);
-        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n, u, w, k8, ok, f, ws, s_x, t,
+        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n, x, w, k8, ok, f, ws, s_x, t,
                                          [] {});
         const int kd = n.E * 4 + D;
         const bool par = (c.ic0 >> D) & 1;
@@ -825,7 +857,6 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
     };
     other(std::integral_constant<int, 1>{});
     other(std::integral_constant<int, 2>{});
-    double u[5];
     T ws2[5];
 #pragma unroll
     for (int iv = 0; iv < 5; ++iv) ws2[iv] = s_x[25 + iv][t];
@@ -835,7 +866,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
     if (__builtin_expect(!all_lanes(ok), 0)) {
         if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, u);
     }
-    finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a.cpart, a.ckeys, a.courant_factor);
+    finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a);
 }
 
 template <int R, bool MIXED, bool EXACT, bool SHARED>

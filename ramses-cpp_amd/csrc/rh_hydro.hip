@@ -2295,7 +2295,7 @@ void launch_form(int variant, const MeshDev& m, const LevelDev& lv, const GasPar
                  double dx, double inv_dx, const FusedCourant& fc, hipStream_t stream) {
     const double* pre = fc.pre_from_uold ? m.uold : m.unew;
     if (takes_dt_by_value(variant, gp, m.ncell)) {
-        StepArgs a{m, lv, gp, d_dt, fc.dt, dx, inv_dx, pre, fc.part, fc.keys, fc.courant_factor};
+        StepArgs a{m, lv, gp, d_dt, fc.dt, dx, inv_dx, pre, fc.part, fc.keys, fc.courant_factor, fc.slots};
         launch_step<R>(MIXED, variant == 6, a, stream);
     } else if (variant == 6) {
         hipLaunchKernelGGL((k_godunov_dims<R, MIXED, EXACT>), dim3((lv.noct + 7) / 8), dim3(192), 0, stream, m, lv,
@@ -2347,6 +2347,11 @@ hipError_t launch_godunov(const MeshDev& m, const LevelDev& lv, const GasParams&
     if ((fc.part || fc.keys) && (variant == 0 || lv.ntgt != 0 || lv.nrec != 0 || lv.nleaf != 8LL * lv.noct))
         return hipErrorInvalidValue;
     if (fc.pre_from_uold && variant == 0) return hipErrorInvalidValue;
+    const CourantSlots& sl = fc.slots;
+    if ((sl.in || sl.out) && (lv.obox || fc.part || !takes_dt_by_value(variant, gp, m.ncell) || lv.ntgt != 0 ||
+                              lv.nrec != 0 || lv.nleaf != 8LL * lv.noct))
+        return hipErrorInvalidValue;
+    if (sl.in && (d_dt || !sl.dt_out)) return hipErrorInvalidValue;
     if (!d_dt && (lv.obox || !takes_dt_by_value(variant, gp, m.ncell))) return hipErrorInvalidValue;
     if ((fc.part && (lv.obox || fc.keys)) || (fc.keys && !lv.obox)) return hipErrorInvalidValue;
     const bool mixed = precision == 1;

@@ -49,6 +49,21 @@ struct GasParams {
     int slope_type, interpol_type;
 };
 
+// Courant minima handed from one step's launch to the next without a
+// reduction between them (a single mesh, where takes_dt_by_value): COURANT_SLOTS
+// ordered keys, COURANT_STRIDE apart, over which the blocks of a launch spread
+// their candidates.  A launch reads its time step from `in` (and stores it in
+// *dt_out), takes its candidates' minima into `out` and refills `clear` with
+// dt_init for the launch after the next.  Any of them may be null.
+constexpr int COURANT_SLOTS = 8, COURANT_STRIDE = 16;
+struct CourantSlots {
+    const unsigned long long* in = nullptr;
+    unsigned long long* out = nullptr;
+    unsigned long long* clear = nullptr;
+    double* dt_out = nullptr;
+    double dt_init = 0.0;
+};
+
 // Launchers (defined in rh_hydro.hip).  All enqueue on `stream`.
 hipError_t launch_set_unew(const MeshDev& m, const LevelDev& lv, hipStream_t stream);
 hipError_t launch_set_uold(const MeshDev& m, const LevelDev& lv, hipStream_t stream);
@@ -123,6 +138,7 @@ struct FusedCourant {
     unsigned long long* keys = nullptr;
     double courant_factor = 0.0;
     double dt = 0.0;  // the time step when d_dt is null (takes_dt_by_value)
+    CourantSlots slots;
 };
 hipError_t launch_godunov(const MeshDev& m, const LevelDev& lv, const GasParams& gp, int riemann, int precision,
                           int variant, const double* d_dt, double dx, double inv_dx, hipStream_t stream,
