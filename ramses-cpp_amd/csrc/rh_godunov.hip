@@ -320,7 +320,7 @@ template <typename T> struct DimFlux {
 // A wave's cells and constants.
 template <typename T> struct Cell {
     int p, ic0, lm, cC;
-    bool leaf;
+    bool leaf, tiny;  // tiny: see fast::prim
     T q[5], y, c2;  // primitives in global order, recip(density), trace_c2
 };
 
@@ -392,14 +392,15 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
         if (i == 1) s = -s;
         dr[i] = s - q[i];
     }
-    fast::prim(u, g, yX, k, ok);
+    bool tiny = c.tiny;
+    fast::prim(u, g, yX, k, ok, tiny);
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
         x[i] = g[rot<D>(i)];
         if (i == 1) x[i] = flip(x[i], sbit);
         dl[i] = q[i] - x[i];
     }
-    fast::prim(w, g, y2, k, ok);
+    fast::prim(w, g, y2, k, ok, tiny);
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
         T z = g[rot<D>(i)];
@@ -407,6 +408,7 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
         dx[i] = x[i] - z;
     }
     Slopes<T, SHARED> sc;
+    fast::keep(dl, dr, k, tiny, ok);
     fast::slopes<T, SHARED, EXACT>(q, dl, dr, c.y, c.c2, slope_type, interpol_type, k, sc);
 
     // X's states on the shared face, from X2, X and C (a coarser X's from its
@@ -418,7 +420,7 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
             int far = par ? rc.y : rc.z;
             if (!coarse || far <= 0) far = n.X;
             load5(m, m.uold, far, u);
-            fast::prim(u, g, y2, k, ok);
+            fast::prim(u, g, y2, k, ok, tiny);
 #pragma unroll
             for (int i = 0; i < 5; ++i) {
                 T z = g[rot<D>(i)];
@@ -429,6 +431,7 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
     }
     {
         Slopes<T, SHARED> sx;
+        fast::keep(dl, dx, k, tiny, ok);
         fast::slopes<T, SHARED, EXACT>(x, dx, dl, yX, fast::trace_c2(x[0], x[4], yX, k), slope_type, interpol_type, k, sx);
         fast::ghost_face<T, SHARED, EXACT>(x, sx, T(1.0), gx, least);
         fast::own_face<T, SHARED, EXACT>(x, sx, T(1.0), om, least);
@@ -715,7 +718,8 @@ RH_DEV void find_cell(const MeshDev& m, const LevelDev& lv, int praw, int t, Cel
     load5(m, m.uold, c.cC, u);
 }
 template <typename T> RH_DEV void take_cell(const double u[5], const Consts<T>& k, Cell<T>& c, bool& ok) {
-    fast::prim(u, c.q, c.y, k, ok);
+    c.tiny = false;
+    fast::prim(u, c.q, c.y, k, ok, c.tiny);
     c.c2 = fast::trace_c2(c.q[0], c.q[4], c.y, k);
 }
 

@@ -189,3 +189,35 @@ def test_courant_of_long_minima_arrays():
                 s.run_uniform(level, dx, 0.8, k)
                 assert s.courant(level, dx, 1.4, 0.8) == dts[k], f"step {k} variant {variant}"
             s.close()
+
+
+@pytest.mark.parametrize("prec,low", [("mixed", 30), ("mixed", 90), ("mixed", 160), ("fp64", 380), ("fp64", 700)])
+@pytest.mark.parametrize("variant", [2, 6])
+@pytest.mark.parametrize("slope_type,interpol_type", [(1, 1), (2, 1), (8, 3), (7, 2), (6, 1)])
+def test_front_velocities(slope_type, interpol_type, variant, prec, low):
+    """Gas nearly at rest, its velocities falling off by orders of magnitude
+    from cell to cell down to 2^-low, as ahead of a front: products of two
+    differences, and in FP32 differences too, vanish."""
+    print(f"case front {prec} low {low} variant {variant} slopes {slope_type} {interpol_type}", flush=True)
+    level = 4
+    m0 = rhydro.uniform_mesh(level)
+    u = m0.state("uold")
+    cells = m0.cells_of_level(level, leaf_only=True)
+    rng = np.random.default_rng(low)
+    x = np.arange(cells.size) // 8 / (cells.size // 8)
+    for i in range(1, 4):
+        e = low * x * rng.uniform(0.7, 1.0, cells.size)
+        u[i, cells] = rng.choice([-1.0, 0.0, 1.0, 1.0, 1.0], cells.size) * rng.uniform(0.5, 1.0, cells.size) * np.exp2(-e)
+    u[0, cells] = np.where(rng.random(cells.size) < 0.3, rng.uniform(0.5, 1.0, cells.size), 1.0)
+    u[4, cells] = 2.5 + 0.5 * (u[1:4, cells] ** 2).sum(0) / u[0, cells]
+    m0.unew[:] = m0.uold
+    kw = dict(gamma=1.4, slope_type=slope_type, interpol_type=interpol_type, riemann="hllc")
+    for dx, dt in ((1.0 / 2 ** level, 1e-2), (1.0 / (3 * 2 ** level), 5e-3)):
+        if prec == "mixed":
+            got, _ = _one_call(m0, level, dx, dt, variant=variant, precision=rhydro.RH_PREC_MIXED, **kw)
+            want, _ = _one_call(m0, level, dx, dt, variant=0, precision=rhydro.RH_PREC_MIXED, **kw)
+        else:
+            got, p = _one_call(m0, level, dx, dt, variant=variant, **kw)
+            want = clone(m0)
+            oracle.OracleMesh(want).godunov_fine(p, level, dt, dx)
+        assert_same(got.unew, want.unew, f"dx {dx}")
