@@ -49,14 +49,14 @@ KERNEL_SOURCES = ["ramses-cpp_amd/csrc/rh_hydro.hip", "ramses-cpp_amd/csrc/rh_go
                   "ramses-cpp_amd/csrc/rh_fast.h", "ramses-cpp_amd/csrc/rh_device.h",
                   "ramses-cpp_amd/csrc/rh_physics.h", "ramses-cpp_amd/csrc/rh_kernels.h", "ramses-cpp_amd/Makefile"]
 PROFILED = {
-    (9, "hllc", 1, 2, "fp64"): {"sources": "aaea3b054087f57a", "traffic": 2172901455,
-                                "valu": {"busy": 0.761, "insts_per_cell": 5941.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 6, "fp64"): {"sources": "aaea3b054087f57a", "traffic": 2175126472,
-                                "valu": {"busy": 0.812, "insts_per_cell": 6237.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 2, "mixed"): {"sources": "aaea3b054087f57a", "traffic": 2197427939,
-                                 "valu": {"busy": 0.849, "insts_per_cell": 3958.2, "courant_epilogue": True}},
-    (9, "hllc", 1, 6, "mixed"): {"sources": "aaea3b054087f57a", "traffic": 2178278029,
-                                 "valu": {"busy": 0.685, "insts_per_cell": 4291.2, "courant_epilogue": True}},
+    (9, "hllc", 1, 2, "fp64"): {"sources": "5dcb27d5d0308185", "traffic": 2187623909,
+                                "valu": {"busy": 0.790, "insts_per_cell": 2695.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 6, "fp64"): {"sources": "5dcb27d5d0308185", "traffic": 2175430086,
+                                "valu": {"busy": 0.634, "insts_per_cell": 2932.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 2, "mixed"): {"sources": "5dcb27d5d0308185", "traffic": 2226339846,
+                                 "valu": {"busy": 0.677, "insts_per_cell": 2165.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 6, "mixed"): {"sources": "5dcb27d5d0308185", "traffic": 2177267133,
+                                 "valu": {"busy": 0.654, "insts_per_cell": 2449.0, "courant_epilogue": True}},
 }
 
 

@@ -95,12 +95,12 @@ template <typename T> struct Consts {
 RH_DEV double e_int(double p, const Consts<double>& k) { return quot(p, k.gm1, k.y_gm1); }
 RH_DEV float e_int(float p, const Consts<float>& k) { return p * k.y_gm1; }
 
-// Upper bound of a state in range (prim).  Within its bounds, and with dt/dx <= 2^20, dt >=
-// 2^-100 (mixed 2^-50), dx in [2^-60, 2^60] and gamma - 1 in [2^-10, 64], no
-// FP64 intermediate of the update exceeds 1e290 and none that is rounded
-// falls below the normal numbers where that could show; the smallest
-// difference of two velocities is 2^-453, so products of two differences do not
-// vanish (FP32: see kept).
+// Upper bound of a state in range (prim).  Within its bounds, and with dt/dx
+// <= 2^20, dt >= 2^-100, dx in [2^-60, 2^60] and gamma - 1 in [2^-10, 64], no
+// FP64 intermediate of the update exceeds 1e290 and none that is rounded falls
+// below the normal numbers where that could show; the smallest difference of
+// two velocities is 2^-453, so products of two differences do not vanish
+// (FP32: see kept).
 constexpr double RANGE_HI = 0x1p50;
 
 // Conservative -> primitive (the operations of ctoprim); y = recip(density).
@@ -141,7 +141,7 @@ RH_DEV void prim(const double ud[5], float q[5], float& y, const Consts<float>& 
     const float s = (v2 + t) + u[0];
     const int least = min(min(__builtin_amdgcn_frexp_expf(q[1]), __builtin_amdgcn_frexp_expf(q[2])),
                           __builtin_amdgcn_frexp_expf(q[3]));
-    ok = ok & (s < (float)RANGE_HI) & (mn(u[0], t) >= 0x1p-20f) & (least > -120);
+    ok = ok & (s < (float)RANGE_HI) & (mn(u[0], t) >= 0x1p-20f);
     tiny = tiny | (least <= -45);
 }
 
@@ -158,8 +158,9 @@ RH_DEV float minmod(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 0.0
 // 20 % of the waves at one step; left to the general path they made the first
 // 40 steps of 48 boxes take 31.9 ms instead of 18.3).  Waves with such
 // velocities take the second difference b through this: 0 where the product
-// vanishes.  Velocities and slopes too small for the face states' exact
-// factors are left to the general form.
+// vanishes.  Slopes too small for the face states' exact factors are left to
+// the general form; of velocities near FP32's smallest a quarter of their
+// source term may differ from the general form's by that smallest number.
 RH_DEV float kept(float a, float b, float lo, bool& ok) {
     const float p = a * b;
     ok = ok & ((p <= 0.0f) | (mn(sabs(a), sabs(b)) >= lo));

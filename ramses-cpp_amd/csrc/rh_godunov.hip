@@ -10,14 +10,16 @@
 // general_cell for the octs of a wave in which some state is out of that
 // frame's range.
 //
-// Bound: the vector ALU, 91-96 % busy.  An HLLC/MinMod update executes about
-// 2,750 VALU instructions per cell in the FP64 form and 2,150 in the mixed form
-// (the kernels of rh_hydro.hip, which select each operand by a cell's place in
-// its oct, round every division separately and trace own and ghost states
-// apart: 5,941 and 3,958); HBM traffic is a quarter of what the memory
-// delivers.  At 2^21 octs (256^3 cells) a launch takes 1.75-1.80 ms in the FP64
-// form and 1.47-1.50 ms in the mixed form, against 3.48 and 2.09 ms; at 512
-// octs 10.0 and 9.1 us against 13.6 and 12.9 us (k_step_dims).
+// Bound: the vector ALU, 79 % (FP64) and 68 % (mixed) busy at the 1.9-2.2 GHz
+// that these launches run at.  An HLLC/MinMod update executes 2,545 VALU
+// instructions per cell in the FP64 form and 2,015 in the mixed form, and 150
+// more for the next step's Courant candidate (the kernels of rh_hydro.hip,
+// which select each operand by a cell's place in its oct, round every division
+// separately and trace own and ghost states apart: 5,747 and 3,779, and
+// 180-195); HBM traffic is a quarter of what the memory delivers.  At 2^21
+// octs (256^3 cells) a launch takes 1.71-1.75 ms in the FP64 form and 1.43-1.45
+// ms in the mixed form, against 3.48 and 2.09 ms; at 512 octs 10.0 and 9.1 us
+// against 13.6 and 12.9 us (k_step_dims).
 // Registers: three waves per SIMD (168 per lane).  Two waves took 2.04 ms
 // against 1.90 (FP64, an earlier order of the code), four waves 1.61 against
 // 1.49 (mixed, 24 bytes spilled): a spill is written through to memory for
@@ -211,24 +213,14 @@ RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& 
     }
 }
 
-// The time step in a launch's slots, for the general path.
-RH_DEV double slots_dt(const unsigned long long* in) {
-    unsigned long long k = in[0];
-#pragma unroll 1
-    for (int i = 1; i < COURANT_SLOTS; ++i) k = min(k, in[i * COURANT_STRIDE]);
-    return key_dt(k);
-}
-
 template <int R, bool MIXED, typename T>
-RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, T (*w)[64], int t, double u[5]) {
+RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, T (*w)[64], int t, double dt, double dx, double u[5]) {
     const MeshDev& m = a.m;
     const LevelDev& lv = a.lv;
     const GasParams& gp = a.gp;
     const Rows<T> W{w, t};
-    double dt, dx = a.dx, inv_dx = a.inv_dx;
-    if (a.d_dt) step_of(lv, p, a.d_dt, dt, dx, inv_dx);
-    else if (a.slots.in) dt = slots_dt(a.slots.in);
-    else dt = a.dt;
+    double inv_dx;
+    if (lv.obox) step_of(lv, p, a.d_dt, dt, dx, inv_dx);  // the wave's are its first oct's
     const double dtdx = dt / dx;
     double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, F[5];
     load_u(a.pre, m.ncell, cC, u);
@@ -619,7 +611,7 @@ RH_DEV bool constants(const StepArgs& a, int p, double& dt, double& dx, Consts<T
     } else {
         k.y_gm1 = uniform((T)(1.0 / a.gp.gm1));
         k.inv = uniform(fast::recip(k.dx));
-        return ok && dt >= 0x1p-50 && dtdx <= 0x1p20 && dx >= 0x1p-40 && dx <= 0x1p40;
+        return ok && dt >= 0x1p-100 && dtdx <= 0x1p20 && dx >= 0x1p-40 && dx <= 0x1p40;
     }
 }
 
@@ -782,7 +774,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
     ok = ok & applies_to(u);
     apply(u, fs, ws, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
     if (__builtin_expect(!all_lanes(ok), 0)) {
-        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, u);
+        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, dt, dx, u);
     }
     finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a);
 }
@@ -868,7 +860,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
     ok = applies_to(u) && !(s_bad[0] | s_bad[1] | s_bad[2]);
     apply(u, fs, ws2, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
     if (__builtin_expect(!all_lanes(ok), 0)) {
-        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, u);
+        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, dt, dx, u);
     }
     finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a);
 }

@@ -3,8 +3,10 @@
 // Kernels (one level per launch unless stated):
 //   k_set_unew / k_set_uold   unew <- uold for every cell of the level's octs /
 //                             uold <- unew for its leaf cells
-//   k_courant_partial/_final  minimum Courant time step over the level's leaf
-//                             cells (wavefront shuffles, block minima, then one
+//   k_courant_partial/_fold/_final
+//                             minimum Courant time step over the level's leaf
+//                             cells (wavefront shuffles, block minima, long
+//                             arrays of them folded by 256 blocks, then one
 //                             1024-thread pass; the first can also do set_unew)
 //   k_step_join               set_uold, the next Courant candidates and
 //                             set_unew in one pass between two steps
@@ -14,7 +16,9 @@
 //   k_godunov                 per-cell form: fluxes, ordered reflux
 //                             accumulation and clamps
 //   k_godunov_oct             oct-in-lanes form of the same update (siblings by
-//                             cross-lane shuffle, ordered accumulation in LDS)
+//                             cross-lane shuffle, ordered accumulation in LDS);
+//                             it and k_godunov_dims serve the launches that the
+//                             step kernels (rh_godunov.hip) do not take
 //   k_coarse_reflux(_wave)    ordered reflux into coarser leaf cells
 //   k_interpol / k_new_octs   prolongation of coarse cells into new octs
 //   k_restrict, k_set_uold_restrict
