@@ -49,14 +49,14 @@ KERNEL_SOURCES = ["ramses-cpp_amd/csrc/rh_hydro.hip", "ramses-cpp_amd/csrc/rh_go
                   "ramses-cpp_amd/csrc/rh_fast.h", "ramses-cpp_amd/csrc/rh_device.h",
                   "ramses-cpp_amd/csrc/rh_physics.h", "ramses-cpp_amd/csrc/rh_kernels.h", "ramses-cpp_amd/Makefile"]
 PROFILED = {
-    (9, "hllc", 1, 2, "fp64"): {"sources": "5dcb27d5d0308185", "traffic": 2187623909,
-                                "valu": {"busy": 0.790, "insts_per_cell": 2695.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 6, "fp64"): {"sources": "5dcb27d5d0308185", "traffic": 2175430086,
-                                "valu": {"busy": 0.634, "insts_per_cell": 2932.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 2, "mixed"): {"sources": "5dcb27d5d0308185", "traffic": 2226339846,
-                                 "valu": {"busy": 0.677, "insts_per_cell": 2165.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 6, "mixed"): {"sources": "5dcb27d5d0308185", "traffic": 2177267133,
-                                 "valu": {"busy": 0.654, "insts_per_cell": 2449.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 2, "fp64"): {"sources": "fb7f48747b7e9448", "traffic": 2187115066,
+                                "valu": {"busy": 0.799, "insts_per_cell": 2689.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 6, "fp64"): {"sources": "fb7f48747b7e9448", "traffic": 2175554237,
+                                "valu": {"busy": 0.635, "insts_per_cell": 2920.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 2, "mixed"): {"sources": "fb7f48747b7e9448", "traffic": 2221442369,
+                                 "valu": {"busy": 0.674, "insts_per_cell": 2148.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 6, "mixed"): {"sources": "fb7f48747b7e9448", "traffic": 2177282211,
+                                 "valu": {"busy": 0.648, "insts_per_cell": 2422.0, "courant_epilogue": True}},
 }
 
 
