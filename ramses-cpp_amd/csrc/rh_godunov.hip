@@ -683,7 +683,8 @@ RH_DEV void finish(const MeshDev& m, const LevelDev& lv, const GasParams& gp, co
         for (int off = 32; off > 0; off >>= 1) w = fast::mx(w, __shfl_xor(w, off, 64));
         if (w > 0.0) cand = (dx / w) * s1 / 1e-4;
     } else {
-        if (leaf) cand = courant_cand_u(m, u, cC, dx, gp.gamma, courant_factor);
+        // dx is the width of the wave's first box; its others have their own.
+        if (leaf) cand = courant_cand_u(m, u, cC, one_box ? dx : lv.box_len[lv.obox[p]], gp.gamma, courant_factor);
         if (one_box) cand = wave_min(cand);
     }
     if (cpart) {
