@@ -27,7 +27,9 @@ template <typename T> RH_DEV void copy5(const T a[5], T b[5]) {
 // as with std::min(dt_max, dt_cand) in the reference loop.
 RH_DEV double min_skip_nan(double a, double b) { return (b < a) ? b : a; }
 
+// A lane's own NaN must not stand for its partners' values either.
 RH_DEV double wave_min(double v) {
+    v = min_skip_nan(__builtin_inf(), v);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         double o = __shfl_xor(v, off, 64);
