@@ -45,6 +45,9 @@ RH_DEV float mn(float a, float b) { return __builtin_fminf(a, b); }
 RH_DEV float mx(float a, float b) { return __builtin_fmaxf(a, b); }
 RH_DEV double fm(double a, double b, double c) { return __builtin_fma(a, b, c); }
 RH_DEV float fm(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// smax(a, 0) that keeps a NaN in FP32 (in range FP64 has none).
+RH_DEV double nonneg(double a) { return mx(a, 0.0); }
+RH_DEV float nonneg(float a) { return smax(a, 0.0f); }
 RH_DEV double signed_as(double a, double s) { return __builtin_copysign(a, s); }
 RH_DEV float signed_as(float a, float s) { return __builtin_copysignf(a, s); }
 
@@ -288,6 +291,18 @@ template <typename T> RH_DEV T face_c2(const T q[5], const Consts<T>& k) {
     return quot(k.gamma * q[4], q[0], recip(q[0]));
 }
 
+// The range of the states does not keep FP32 products from overflowing (ar*p
+// from densities of about 2^30 with sound speeds of 2^20, and sooner where a
+// long time step takes the face states beyond the cells').  The general solver
+// may return something finite there -- HLLC a physical flux where this one
+// multiplies an infinite star term by 0 -- and its minima and maxima treat a
+// NaN differently, so fluxes that are not finite are left to it: seen gathers
+// the fluxes and stays infinite or NaN once one is.
+RH_DEV void watch(const double*, double&) {}
+RH_DEV void watch(const float F[5], float& seen) { seen = fm(F[0], F[1], fm(F[2], F[3], seen)) + F[4]; }
+RH_DEV bool finite(double) { return true; }
+RH_DEV bool finite(float seen) { return sabs(seen) < __builtin_inff(); }
+
 // riemann_hllc.  Its floors on densities, pressures, sound speeds and the
 // contact speed are left to the general form: ok is cleared where one would
 // apply (a pressure below density*smallp has a squared sound speed of at most
@@ -303,7 +318,7 @@ template <typename T> RH_DEV void hllc(const T l[5], const T r[5], T F[5], const
     const T div = ar + al;
     const T yd = recip(div);
     const T us = quot((ar * r[1] + al * l[1]) + (l[4] - r[4]), div, yd);
-    const T ps = mx(quot((ar * l[4] + al * r[4]) + al * ar * (l[1] - r[1]), div, yd), T(0.0));
+    const T ps = nonneg(quot((ar * l[4] + al * r[4]) + al * ar * (l[1] - r[1]), div, yd));
     ok = ok & (mn(c2l, c2r) >= T(2e-20)) & (sabs(us) <= T(1e6));
     const bool pass_l = sl > T(0.0), pass_r = sr < T(0.0);
     const bool left = pass_l | (!pass_r & ((us > T(0.0)) | (mir & (us == T(0.0)))));

@@ -437,6 +437,9 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
     // X's own flux through the shared face.
     fast::ghost_face<T, SHARED, EXACT>(q, sc, T(-1.0), l, least);
     fast::riemann<R>(om, l, F, k, par, ok);
+    T seen = T(0);
+    fast::watch(F, seen);  // the cell's own fluxes: applies_to
+    ok = ok & fast::finite(seen);
 #pragma unroll
     for (int i = 0; i < 5; ++i) s_x[5 * D + rot<D>(i)][t] = contribution(F[i], k8, i == 1 ? sbit : 0);
     // The cell's own.
@@ -522,9 +525,12 @@ RH_DEV void own_update_fast(double u[5], const double fs[5], double dtdx, const 
     u[4] = fast::mn(u[4], d * 1e8);
 }
 // Whether the state an update starts from is finite and no larger than 2^100
-// (it is uold's, already in range, except where a caller has changed unew).
-RH_DEV bool applies_to(const double u[5]) {
-    return ((fabs(u[0]) + fabs(u[1])) + (fabs(u[2]) + fabs(u[3]))) + fabs(u[4]) < 0x1p100;
+// (it is uold's, already in range, except where a caller has changed unew),
+// and in the mixed form what its fluxes add to it too (fast::watch).
+template <typename T> RH_DEV bool applies_to(const double u[5], const double fs[5]) {
+    double s = ((fabs(u[0]) + fabs(u[1])) + (fabs(u[2]) + fabs(u[3]))) + fabs(u[4]);
+    if constexpr (sizeof(T) == 4) s += ((fabs(fs[0]) + fabs(fs[1])) + (fabs(fs[2]) + fabs(fs[3]))) + fabs(fs[4]);
+    return s < 0x1p100;
 }
 
 // Wave speed sum of the Courant candidate, courant_cand_u() up to u_wave, for
@@ -772,7 +778,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
     pass(std::integral_constant<int, 1>{});
     pass(std::integral_constant<int, 2>{});
     const int key[3] = {n[0].E * 4, n[1].E * 4 + 1, n[2].E * 4 + 2};
-    ok = ok & applies_to(u);
+    ok = ok & applies_to<T>(u, fs);
     apply(u, fs, ws, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
     if (__builtin_expect(!all_lanes(ok), 0)) {
         if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, dt, dx, u);
@@ -858,7 +864,7 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
 #pragma unroll
     for (int iv = 0; iv < 5; ++iv) ws2[iv] = s_x[25 + iv][t];
     load5(m, a.pre, c.cC, u);
-    ok = applies_to(u) && !(s_bad[0] | s_bad[1] | s_bad[2]);
+    ok = applies_to<T>(u, fs) && !(s_bad[0] | s_bad[1] | s_bad[2]);
     apply(u, fs, ws2, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
     if (__builtin_expect(!all_lanes(ok), 0)) {
         if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, dt, dx, u);
