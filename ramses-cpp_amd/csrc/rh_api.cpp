@@ -705,6 +705,14 @@ int rh_interpol_hydro(rh_ctx* c, int n_octs, const double* u1, double* u2) {
             RH_HIP(c, hipHostMalloc((void**)&c->h_interpol, (size_t)cap * 75 * sizeof(double), hipHostMallocDefault));
             c->interpol_cap = cap;
         }
+        // Operands and results may share memory: a later batch's operands must
+        // not be read after an earlier one's results are written.
+        std::vector<double> kept;
+        const size_t n1 = (size_t)n_octs * 7 * 64, n2 = (size_t)n_octs * 8 * 64;
+        if (n_octs > batch && u1 < u2 + n2 && u2 < u1 + n1) {
+            kept.assign(u1, u1 + n1);
+            u1 = kept.data();
+        }
         for (int o0 = 0; o0 < n_octs; o0 += batch) {
             const int n = std::min(batch, n_octs - o0);
             double* in = c->h_interpol;
