@@ -57,210 +57,390 @@ using fast::flip;
 using fast::Slopes;
 
 // ---------------------------------------------------------------------------
-// General form of one cell's update: any finite or non-finite state, any mesh.
-// One lane does one cell on its own, with the routines of rh_physics.h.  It
-// is reached by waves that hold a state out of range or an oct that is its
-// own neighbour, so it is written for few registers and little code, not for
-// speed: one face flux at a time, the incoming ones recomputed in the order
-// they are applied, states and slopes in the lane's column of LDS (w, the 25
-// rows that the ordinary form keeps its contributions in) and the components
-// taken one after another.  Held to the registers of the ordinary form it
-// costs waves in range nothing; with its states in registers the kernel
-// spilled in the ordinary form too (FP64 1.77 ms per launch at 2^21 octs
-// became 1.84).
-template <typename T> struct Rows {
-    T (*w)[64];
-    int t;
-    RH_DEV T& operator()(int row) const { return w[row][t]; }
+// General form of a wave's update: any finite or non-finite state, any mesh,
+// octs of several boxes, each lane with its own time step and cell width.  The
+// routines of rh_physics.h in the reference's orientation, the eight cells of
+// an oct in eight lanes as in the ordinary form: per dimension four traces and
+// three Riemann problems a cell.  It is reached by waves that hold a state out
+// of range (ahead of a blast's front, where velocities fall off towards 0; cold
+// gas in the mixed form) or an oct that is its own neighbour.
+// Bound: a launch waits for its slowest wave, so what counts is the length of
+// one wave's instruction stream, and where many waves come here, spills, which
+// are written to memory.  k_step_dims has each of its waves do its own
+// dimension.  One such wave in a launch of 512 octs adds 8 us in the FP64 form
+// and 6 in the mixed form, in one of 32,768 octs 20 and 7; with every wave
+// here 2^18 octs take 0.70 and 0.26 ms.  (One lane per cell, recomputing the
+// face problems one after another from LDS, added 87 and 71 us, 82 and 67, and
+// took 1.55 and 1.12 ms: 64^3 blasts ran at 112 instead of 56 us per step.)
+
+template <typename T> using SharedRows = __attribute__((address_space(3))) T*;
+template <typename T, int N> RH_DEV SharedRows<T> shared_rows(T (*w)[N]) { return (SharedRows<T>)&w[0][0]; }
+
+// The launch's arguments, read again: kept in registers through the ordinary
+// form they would cost it some.
+RH_DEV const void* launch_args() { return (const void*)__builtin_amdgcn_kernarg_segment_ptr(); }
+RH_DEV StepArgs args_at(const void* p) {
+    typedef const __attribute__((address_space(4))) char* Kernarg;
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned long long u = ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+                                 (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+    StepArgs a;
+    __builtin_memcpy(&a, (const void*)(Kernarg)u, sizeof(a));
+    return a;
+}
+
+// A value that is the same in every lane, in scalar registers.
+RH_DEV double uniform(double x) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+RH_DEV float uniform(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
+
+// Five rows of a lane's column.
+template <typename T> RH_DEV void put_rows(SharedRows<T> w, int t, const T v[5]) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) w[i * 64 + t] = v[i];
+}
+template <typename T> RH_DEV void get_rows(SharedRows<T> w, int t, T v[5]) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) v[i] = w[i * 64 + t];
+}
+
+// A lane's cell.
+struct GeneralCell {
+    int p, ic0, lm, cC;
+    bool leaf;
 };
-constexpr int ROW_C = 0, ROW_N = 5, ROW_O = 10, ROW_SC = 15, ROW_SN = 20;
-
-// Rotated primitives of a cell into rows `to`; rows `fallback` where there is
-// no cell.
+// The step of its box.
+template <typename T> struct GeneralStep {
+    double dtdx;
+    T dt, dx, inv;  // inv: 1/dx where exact
+};
+// In the FP64 form nothing is moved across.
+template <bool MIXED> RH_DEV void phase() {
+    if constexpr (!MIXED) __builtin_amdgcn_sched_barrier(0);
+}
 template <typename T>
-RH_DEV void general_prim(const MeshDev& m, const GasParams& gp, const Gas<T>& gc, int icell, int d, int fallback, int to,
-                         const Rows<T>& W) {
-    if (icell > 0) {
-        const Gas<double> gd{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1};
-        double u[5];
-        T q[5];
-        load_u(m.uold, m.ncell, icell, u);
-        face_prim(u, q, gd, gc);
-        rotate(q, d);
-#pragma unroll
-        for (int i = 0; i < 5; ++i) W(to + i) = q[i];
-    } else {
-#pragma unroll 1
-        for (int i = 0; i < 5; ++i) W(to + i) = W(fallback + i);
-    }
+RH_DEV void general_prim(const StepArgs& a, const Gas<T>& gc, int icell, T q[5]) {
+    const Gas<double> gd{a.gp.gamma, a.gp.gm1, a.gp.smalle, a.gp.smallp, 1.0 / a.gp.gm1};
+    double u[5];
+    load_u(a.m.uold, a.m.ncell, icell, u);
+    face_prim(u, q, gd, gc);
+}
+RH_DEV GeneralCell general_cell(const StepArgs& a, int praw, int t) {
+    GeneralCell c;
+    c.ic0 = t & 7;
+    c.p = min(praw, a.lv.noct - 1);
+    c.lm = a.lv.leaf[c.p];
+    c.leaf = praw < a.lv.noct && ((c.lm >> c.ic0) & 1);
+    c.cC = cell_id(a.m, a.lv.grid[c.p], c.ic0);
+    return c;
+}
+template <typename T> RH_DEV GeneralStep<T> general_step(const StepArgs& a, int p, double dt, double dx) {
+    double inv_dx = a.inv_dx;
+    if (a.lv.obox) step_of(a.lv, p, a.d_dt, dt, dx, inv_dx);
+    return {dt / dx, (T)dt, (T)dx, (T)inv_dx};
+}
+template <typename T> RH_DEV Gas<T> general_gas(const StepArgs& a) {
+    return {(T)a.gp.gamma, (T)a.gp.gm1, (T)a.gp.smalle, (T)a.gp.smallp, (T)(1.0 / a.gp.gm1)};
 }
 
-// The face state, on the side given (upper: towards the right neighbour), of
-// the cell in rows q with left and right neighbours in rows a and c, into rows
-// `to`: its own (slope_type) or its ghost state (interpol_type).  The
-// operations of own_slopes / ghost_slopes and trace.
-template <typename T>
-RH_DEV void general_state(const GasParams& gp, const Gas<T>& gc, T dt, T dx, int a, int q, int c, bool own, bool upper,
-                          int to, const Rows<T>& W) {
-    const Len<T, false> lo{dx, T(0)};
-    const Len<T, false> len = own ? lo : coarse(lo);
-    const int st = gp.slope_type;
-    const T nu = over(W(q + 1) * dt, lo);
-#pragma unroll 1
-    for (int i = 0; i < 5; ++i) {
-        const T qa = W(a + i), qb = W(q + i), qc = W(c + i);
-        T lim;
-        if (own) lim = (st == 0 || ((st == 5 || st == 6) && i != 0)) ? T(0.0) : limiter(qa, qb, qc, st, nu);
-        else lim = ghost_limiter(qb - qa, qc - qb, gp.interpol_type);
-        W(to + i) = (own && (st == 0 || ((st == 5 || st == 6) && i != 0))) ? T(0.0) : over(lim, len);
-    }
-    const T dr = W(to), du = W(to + 1), dp = W(to + 4);
-    const T r = smax(W(q), T(1e-10)), u = W(q + 1);
-    const T c2 = cs2(r, smax(W(q + 4), r * T(1e-20)), gc);
-    const T s0 = -u * dr - du * r, s1 = -u * du - dv(dp, r), s4 = -u * dp - du * r * c2;
-    const T hdx = T(0.5) * len.dx, hdt = T(0.5) * dt;
-#pragma unroll 1
-    for (int i = 0; i < 5; ++i) {
-        const T step = hdx * W(to + i), src = i == 0 ? s0 : i == 1 ? s1 : i == 4 ? s4 : T(0);
-        T v = (upper ? W(q + i) + step : W(q + i) - step) + hdt * src;
-        if (i == 0 && v < T(1e-10)) v = r;
-        W(to + i) = v;
-    }
-}
-
-// One face flux of a cell, its own through face f or, incoming, the one its
-// neighbour there computes for the shared face (0 where there is none).
-template <int R, bool MIXED, typename T>
-RH_DEV void general_flux(const MeshDev& m, const LevelDev& lv, const GasParams& gp, int p, int ic0, int cC, double dt,
-                         double dx, int f, bool incoming, const Rows<T>& W, double Fd[5]) {
-    const Gas<T> gc{(T)gp.gamma, (T)gp.gm1, (T)gp.smalle, (T)gp.smallp, (T)(1.0 / gp.gm1)};
-    const T dtc = (T)dt, dxc = (T)dx;
-    const int d = f >> 1, side = f & 1, b = 1 << d, par = (ic0 >> d) & 1;
-#pragma unroll
-    for (int iv = 0; iv < 5; ++iv) Fd[iv] = 0.0;
-    // The neighbour X across the cell's oct face (in oct E, or a record) and
-    // its sibling S.
-    const int E = lv.nbo[(size_t)(2 * d + par) * lv.noct + p];
+// One dimension: the cell's own fluxes through the oct's face (Fe) and towards
+// its sibling (Fi), and the flux X computes through the oct's face (Fx);
+// rotated order, zero where there is none.  w: five rows for what does not fit
+// the registers.
+template <int R, bool MIXED, bool EXACT, bool SHARED, typename T>
+RH_DEV void general_dim(const StepArgs& a, const Gas<T>& gc, const GeneralCell& c, GeneralStep<T> g, int d,
+                        SharedRows<T> w, int t, T Fe[5], T Fi[5], T Fx[5]) {
+    const MeshDev& m = a.m;
+    const LevelDev& lv = a.lv;
+    const int st = SHARED ? 1 : a.gp.slope_type, it = SHARED ? 1 : a.gp.interpol_type;
+    const Gas<double> gd{a.gp.gamma, a.gp.gm1, a.gp.smalle, a.gp.smallp, 1.0 / a.gp.gm1};
+    // Nothing made of them is kept from one dimension to the next.
+    if constexpr (!MIXED) asm volatile("" : "+v"(g.dt), "+v"(g.dx));
+    const Len<T, EXACT> len{g.dx, g.inv};
+    // trace() of a cell's own (over dx) or ghost state (over twice that).
+    auto traced = [&](const T q[5], const T dq[5], T hdx, T qm[5], T qp[5]) {
+        const T r = smax(q[0], T(1e-10));
+        trace_core(q, dq, r, q[1], cs2(r, smax(q[4], r * T(1e-20)), gc), hdx, T(0.5) * g.dt, qm, qp);
+    };
+    const int b = 1 << d;
+    const bool par = (c.ic0 >> d) & 1;
+    const int icS = c.ic0 ^ b;
+    const int E = lv.nbo[(size_t)(2 * d + (par ? 1 : 0)) * lv.noct + c.p];
     int4 rc = make_int4(0, 0, 0, 0);
-    int X;
-    if (E >= 0) X = cell_id(m, lv.grid[E], ic0 ^ b);
-    else {
+    int X, X2 = 0, cC = c.cC;
+    if (E >= 0) {
+        const int gE = lv.grid[E];
+        X = cell_id(m, gE, icS);
+        if ((lv.leaf[E] >> icS) & 1) X2 = cell_id(m, gE, c.ic0);
+    } else {
         rc = lv.rec[-1 - E];
         X = rc.x;
     }
-    const int S = cell_id(m, lv.grid[p], ic0 ^ b);
-    const bool across = side == par;  // this face is the oct's face
-    // The cell beyond the neighbour N across the face, and whether N is there
-    // to solve with.
-    int beyond;
-    bool solve, reflux = false, bound = false;
-    if (!across) {
-        solve = (lv.leaf[p] >> (ic0 ^ b)) & 1;
-        const int E2 = lv.nbo[(size_t)(2 * d + 1 - par) * lv.noct + p];
-        beyond = E2 >= 0 ? cell_id(m, lv.grid[E2], ic0) : lv.rec[-1 - E2].x;
-    } else if (E >= 0) {
-        solve = (lv.leaf[E] >> (ic0 ^ b)) & 1;
-        beyond = cell_id(m, lv.grid[E], ic0);
-    } else {
-        solve = !incoming && !(rc.w & REC_REFINED_DEV);
-        bound = rc.w & REC_BOUNDARY_DEV;
-        reflux = solve && !bound;
-        beyond = side ? rc.z : rc.y;
+    // The FP64 form's phases are kept apart: scheduled into one another they need
+    // more registers than there are, and every spill is written to memory.
+    T q[5], x[5];
+    general_prim(a, gc, c.cC, q);
+    copy5(q, x);
+    if (X > 0) general_prim(a, gc, X, x);
+    rotate(q, d);
+    rotate(x, d);
+    phase<MIXED>();
+    // The cell's ghost and own states: towards X (gx, ox) and towards the
+    // sibling (l, z, of which the sibling's own ghost state comes here).
+    T ox[5], gx[5], l[5], r[5], z[5], mi[5], pl[5];
+    {
+        T s[5], dq[5];
+        shfl5(q, s, b);
+        sel5(par, s, x, l);
+        sel5(par, x, s, r);
+        ghost_slopes(l, q, r, it, coarse(len), dq);
+        phase<MIXED>();
+        traced(q, dq, g.dx, mi, pl);
+        sel5(par, mi, pl, gx);
+        if constexpr (!MIXED) put_rows(w, t, gx);
+        sel5(par, pl, mi, z);
+        phase<MIXED>();
+        own_slopes(l, q, r, st, g.dt, len, dq);
+        phase<MIXED>();
+        traced(q, dq, T(0.5) * g.dx, mi, pl);
+        sel5(par, mi, pl, ox);
+        sel5(par, pl, mi, s);
+        shfl5(z, z, b);
+        sel5(par, z, s, l);
+        sel5(par, s, z, r);
     }
-    if (!solve) return;
-    general_prim(m, gp, gc, cC, d, ROW_C, ROW_C, W);
-    general_prim(m, gp, gc, across ? X : S, d, ROW_C, ROW_N, W);
-    general_prim(m, gp, gc, across ? S : X, d, ROW_C, ROW_O, W);
-    general_state(gp, gc, dtc, dxc, side ? ROW_O : ROW_N, ROW_C, side ? ROW_N : ROW_O, !incoming, side != 0, ROW_SC, W);
-    if (bound) {
+    phase<MIXED>();
+    solve_face<R, MIXED>(l, r, Fi, gc, gd);
+    phase<MIXED>();
+    const bool sib_leaf = (c.lm >> icS) & 1;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        Fi[i] = sib_leaf ? Fi[i] : T(0);
+        Fe[i] = Fx[i] = T(0);
+    }
+
+    // The neighbour's states on the oct's face: z its ghost state, x its own.
+    const bool refined = rc.w & REC_REFINED_DEV, bound = rc.w & REC_BOUNDARY_DEV;
+    if (E >= 0 ? X2 <= 0 : refined) return;
+    if constexpr (!MIXED) {
+        // Read again: kept through the solve they would be spilled.
+        asm volatile("" : "+v"(X), "+v"(cC)::"memory");
+        if (!bound) {
+            general_prim(a, gc, X > 0 ? X : cC, x);
+            rotate(x, d);
+        }
+        if (E >= 0) {
+            general_prim(a, gc, cC, q);
+            rotate(q, d);
+        }
+    }
+    if (E >= 0) {
+        T dq[5];
+        general_prim(a, gc, X2, r);
+        rotate(r, d);
+        sel5(par, q, r, l);
+        sel5(par, r, q, r);
+        phase<MIXED>();
+        ghost_slopes(l, x, r, it, coarse(len), dq);
+        phase<MIXED>();
+        traced(x, dq, g.dx, mi, pl);
+        sel5(par, pl, mi, z);
+        phase<MIXED>();
+        own_slopes(l, x, r, st, g.dt, len, dq);
+        phase<MIXED>();
+        traced(x, dq, T(0.5) * g.dx, mi, pl);
+        sel5(par, pl, mi, x);
+    } else if (bound) {
         // The cell's own state with the normal momentum reversed, traced
         // without slopes.
-        const Gas<double> gd{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1};
         double u[5];
         load_u(m.uold, m.ncell, cC, u);
 #pragma unroll
         for (int i = 1; i <= 3; ++i)
             if (i == 1 + d) u[i] = u[i] * -1.0;
-        T q[5], qm[5], qp[5], dq[5] = {T(0), T(0), T(0), T(0), T(0)};
+        T dq[5] = {T(0), T(0), T(0), T(0), T(0)};
         face_prim(u, q, gd, gc);
         rotate(q, d);
-        trace(q, dq, dtc, dxc, qm, qp, gc);
-#pragma unroll
-        for (int i = 0; i < 5; ++i) W(ROW_SN + i) = side ? qp[i] : qm[i];
+        traced(q, dq, T(0.5) * g.dx, mi, pl);
+        sel5(par, pl, mi, z);
     } else {
-        // N's far neighbour and, on this side, the cell (a coarser N's own
-        // neighbour where N is a record).
-        general_prim(m, gp, gc, beyond, d, ROW_N, ROW_O, W);
-        if (reflux) general_prim(m, gp, gc, side ? rc.y : rc.z, d, ROW_N, ROW_C, W);
-        general_state(gp, gc, dtc, dxc, side ? ROW_C : ROW_O, ROW_N, side ? ROW_O : ROW_C, incoming, side == 0, ROW_SN,
-                      W);
+        // A coarser cell, between its own neighbours.
+        copy5(x, l);
+        copy5(x, r);
+        if (rc.y > 0) {
+            general_prim(a, gc, rc.y, l);
+            rotate(l, d);
+        }
+        if (rc.z > 0) {
+            general_prim(a, gc, rc.z, r);
+            rotate(r, d);
+        }
+        T dq[5];
+        ghost_slopes(l, x, r, it, coarse(len), dq);
+        traced(x, dq, g.dx, mi, pl);
+        sel5(par, pl, mi, z);
     }
-    T l[5], r[5], F[5];
+    phase<MIXED>();
+    sel5(par, ox, z, l);
+    sel5(par, z, ox, r);
+    solve_face<R, MIXED>(l, r, Fe, gc, gd);
+    phase<MIXED>();
+    if (E >= 0) {
+        if constexpr (!MIXED) get_rows(w, t, gx);
+        sel5(par, gx, x, l);
+        sel5(par, x, gx, r);
+        solve_face<R, MIXED>(l, r, Fx, gc, gd);
+    } else if (!bound && c.leaf) {
+        const int slot = lv.rec_slot[-1 - E] + face_slot(c.ic0, d);
+        const double sg = par ? -1.0 : 1.0;
+        T F[5];
+        rotated(Fe, F, d);
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        l[i] = W((side ? ROW_SC : ROW_SN) + i);
-        r[i] = W((side ? ROW_SN : ROW_SC) + i);
+        for (int iv = 0; iv < 5; ++iv) lv.slot_r[(size_t)slot * 5 + iv] = g.dtdx * sg * F[iv] * 0.125;
     }
-    solve_face<R, MIXED>(l, r, F, gc, Gas<double>{gp.gamma, gp.gm1, gp.smalle, gp.smallp, 1.0 / gp.gm1});
-    rotate(F, d);
+    phase<MIXED>();
+}
+
+// Contribution rows as the ordinary form keeps them (see contribution()): what
+// is added to the cell, the mixed form's without its factor.
+RH_DEV double general_row(double F, double dtdx, bool minus) { return dtdx * (minus ? -F : F) * 0.125; }
+RH_DEV float general_row(float F, double, bool minus) { return minus ? -F : F; }
+RH_DEV double general_added(double w, double) { return w; }
+RH_DEV double general_added(float w, double dtdx) { return dtdx * (double)w * 0.125; }
+template <typename T>
+RH_DEV void general_rows(const T F[5], int d, double dtdx, bool minus, T out[5]) {
+    rotated(F, out, d);
 #pragma unroll
-    for (int iv = 0; iv < 5; ++iv) Fd[iv] = (double)F[iv];
-    if (reflux) {
-        const int slot = lv.rec_slot[-1 - E] + face_slot(ic0, d);
-        const double sg = side ? -1.0 : 1.0;
+    for (int iv = 0; iv < 5; ++iv) out[iv] = general_row(out[iv], dtdx, minus);
+}
+
+// The ordered accumulation of a cell: its own update takes its place among the
+// contributions by their keys.  w: rows 5d+iv from X of dimension d, rows
+// 15+5d+iv from S of dimensions 0 and 1; ws2 those of dimension 2.
+template <typename T>
+RH_DEV void general_apply(const StepArgs& a, const GeneralCell& c, double dtdx, double u[5], const double fs[5], const T ws2[5],
+                          SharedRows<T> w, int t) {
+    long long kin[6];
+    incoming_keys(a.lv, c.p, c.ic0, c.lm, kin);
+    const long long KOWN = ((long long)c.p * 8 + c.ic0) * 8 + 6;
+    int done = 0;
+#pragma unroll 1
+    for (int step = 0; step < 7; ++step) {
+        long long best = (done & 64) ? KMAX : KOWN;
+        int f = (done & 64) ? 7 : 6;
 #pragma unroll
-        for (int iv = 0; iv < 5; ++iv) lv.slot_r[(size_t)slot * 5 + iv] = dt / dx * sg * Fd[iv] * 0.125;
+        for (int j = 0; j < 6; ++j) {
+            const bool take = !((done >> j) & 1) && kin[j] >= 0 && kin[j] < best;
+            best = take ? kin[j] : best;
+            f = take ? j : f;
+        }
+        if (f == 7) break;
+        done |= 1 << f;
+        if (f == 6) {
+            own_update(u, fs, dtdx, a.gp);
+        } else {
+            // Face f of the cell is the one across which X lies where its
+            // side is the cell's side of the oct.
+            const int d = f >> 1;
+            const bool from_x = (f & 1) == ((c.ic0 >> d) & 1), in_regs = f >= 4 && !from_x;
+            const int row = from_x ? 5 * d : 15 + 5 * (d & 1);
+#pragma unroll
+            for (int iv = 0; iv < 5; ++iv) {
+                const T v = w[(row + iv) * 64 + t];
+                u[iv] = u[iv] + general_added(in_regs ? ws2[iv] : v, dtdx);
+            }
+        }
     }
 }
 
-template <int R, bool MIXED, typename T>
-RH_DEV void general_cell(const StepArgs& a, int p, int ic0, int cC, T (*w)[64], int t, double dt, double dx, double u[5]) {
-    const MeshDev& m = a.m;
-    const LevelDev& lv = a.lv;
-    const GasParams& gp = a.gp;
-    const Rows<T> W{w, t};
-    double inv_dx;
-    if (lv.obox) step_of(lv, p, a.d_dt, dt, dx, inv_dx);  // the wave's are its first oct's
-    const double dtdx = dt / dx;
-    double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, F[5];
-    load_u(a.pre, m.ncell, cC, u);
-    const long long KOWN = ((long long)p * 8 + ic0) * 8 + 6;
-    int done = 0;
-    // Six own fluxes in face order, then the contributions in key order with
-    // the cell's own update among them.
-#pragma unroll 1
-    for (int it = 0; it < 13; ++it) {
-        asm volatile("" : "+v"(p), "+v"(ic0), "+v"(cC)::"memory");  // nothing is kept from one face to the next
-        int f = it;
-        if (it >= 6) {
-            long long kin[6];
-            incoming_keys(lv, p, ic0, lv.leaf[p], kin);
-            long long best = (done & 64) ? KMAX : KOWN;
-            f = (done & 64) ? 7 : 6;
+template <bool MIXED> using StepType = std::conditional_t<MIXED, float, double>;
+
+// The whole update of a wave: the new state of its cells.  praw: the lane's
+// oct; w: 25 rows.
+template <int R, bool MIXED, bool EXACT, bool SHARED>
+RH_DEV void general_wave(const void* args, SharedRows<StepType<MIXED>> w, int praw, int t, double dt, double dx,
+                         double u[5]) {
+    using T = StepType<MIXED>;
+    const StepArgs a = args_at(args);
+    const Gas<T> gc = general_gas<T>(a);
+    const GeneralCell c = general_cell(a, praw, t);
+    const GeneralStep<T> g = general_step<T>(a, c.p, dt, dx);
+    double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    T ws[5];
+    // As in k_godunov_oct: three copies of the dimension's code lose more in
+    // instruction fetch than the constant rotations gain in the FP64 form
+    // of HLLC only.
+    constexpr int DIM_UNROLL = (MIXED || R != 2) ? 3 : 1;
+#pragma unroll DIM_UNROLL
+    for (int d = 0; d < 3; ++d) {
+        T Fe[5], Fi[5], Fx[5], row[5];
+        general_dim<R, MIXED, EXACT, SHARED>(a, gc, c, g, d, w + 5 * d * 64, t, Fe, Fi, Fx);
+        const bool par = (c.ic0 >> d) & 1;
+        general_rows(Fx, d, g.dtdx, par, row);
+        put_rows(w + 5 * d * 64, t, row);
+        shfl5(Fi, row, 1 << d);
+        general_rows(row, d, g.dtdx, !par, ws);
+        if (d < 2) put_rows(w + (15 + 5 * d) * 64, t, ws);
+        rotate(Fe, d);
+        rotate(Fi, d);
 #pragma unroll
-            for (int j = 0; j < 6; ++j) {
-                const bool take = !((done >> j) & 1) && kin[j] >= 0 && kin[j] < best;
-                best = take ? kin[j] : best;
-                f = take ? j : f;
-            }
-            if (f == 7) break;
-            done |= 1 << f;
-            if (f == 6) {
-                own_update(u, fs, dtdx, gp);
-                continue;
-            }
-        }
-        general_flux<R, MIXED>(m, lv, gp, p, ic0, cC, dt, dx, f, it >= 6, W, F);
-        if (it < 6) {
-            const double sg = (f & 1) ? -1.0 : 1.0;
-#pragma unroll
-            for (int iv = 0; iv < 5; ++iv) fs[iv] = fs[iv] + sg * F[iv];
-        } else {
-            const double sdt = dtdx * ((f & 1) ? 1.0 : -1.0);
-#pragma unroll
-            for (int iv = 0; iv < 5; ++iv) u[iv] = u[iv] - sdt * F[iv] * 0.125;
+        for (int iv = 0; iv < 5; ++iv) {
+            fs[iv] = fs[iv] + (double)(par ? Fi[iv] : Fe[iv]);
+            fs[iv] = fs[iv] - (double)(par ? Fe[iv] : Fi[iv]);
         }
     }
+    load_u(a.pre, a.m.ncell, c.cC, u);
+    if (c.leaf) general_apply(a, c, g.dtdx, u, fs, ws, w, t);
+}
+
+// One dimension for k_step_dims, with the results where dim_pass leaves its
+// own: contributions in rows 5d and 15+5d of w, own fluxes in the cell's frame
+// (rh_fast.h) in rows 0-4 and 5-9 of o.
+template <int R, bool MIXED, bool EXACT, bool SHARED>
+__device__ __attribute__((noinline)) void general_one_dim(const void* args, SharedRows<StepType<MIXED>> w,
+                                                          SharedRows<StepType<MIXED>> o, int d, int praw, int t,
+                                                          double dt, double dx) {
+    using T = StepType<MIXED>;
+    const StepArgs a = args_at(args);
+    d = __builtin_amdgcn_readfirstlane(d);
+    const Gas<T> gc = general_gas<T>(a);
+    const GeneralCell c = general_cell(a, praw, t);
+    const GeneralStep<T> g = general_step<T>(a, c.p, dt, dx);
+    T Fe[5], Fi[5], Fx[5], row[5];
+    general_dim<R, MIXED, EXACT, SHARED>(a, gc, c, g, d, w + 5 * d * 64, t, Fe, Fi, Fx);
+    const bool par = (c.ic0 >> d) & 1;
+    general_rows(Fx, d, g.dtdx, par, row);
+    put_rows(w + 5 * d * 64, t, row);
+    shfl5(Fi, Fx, 1 << d);
+    general_rows(Fx, d, g.dtdx, !par, row);
+    put_rows(w + (15 + 5 * d) * 64, t, row);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        Fe[i] = par && i != 1 ? -Fe[i] : Fe[i];
+        Fi[i] = par && i != 1 ? -Fi[i] : Fi[i];
+    }
+    put_rows(o, t, Fe);
+    put_rows(o + 5 * 64, t, Fi);
+}
+// The accumulation for k_step_dims (row 25: those of S of dimension 2).
+struct State5 {
+    double u[5];
+};
+template <bool MIXED>
+__device__ __attribute__((noinline)) State5 general_sum(const void* args, SharedRows<StepType<MIXED>> w, State5 fs,
+                                                        int praw, int t, double dt, double dx) {
+    using T = StepType<MIXED>;
+    const StepArgs a = args_at(args);
+    const GeneralCell c = general_cell(a, praw, t);
+    State5 s;
+    const GeneralStep<T> g = general_step<T>(a, c.p, dt, dx);
+    T ws2[5];
+    get_rows(w + 25 * 64, t, ws2);
+    load_u(a.pre, a.m.ncell, c.cC, s.u);
+    if (c.leaf) general_apply(a, c, g.dtdx, s.u, fs.u, ws2, w, t);
+    return s;
 }
 
 // ---------------------------------------------------------------------------
@@ -399,6 +579,8 @@ RH_DEV void dim_pass(const MeshDev& m, const LevelDev& lv, int slope_type, int i
         if (i == 1) z = flip(z, sbit);
         dx[i] = x[i] - z;
     }
+    // A wave with a state out of range has nothing to gain from the rest.
+    if (__builtin_expect(!all_lanes(ok), 0)) return;
     Slopes<T, SHARED> sc;
     fast::keep(dl, dr, k, tiny, ok);
     fast::slopes<T, SHARED, EXACT>(q, dl, dr, c.y, c.c2, slope_type, interpol_type, k, sc);
@@ -570,11 +752,6 @@ RH_DEV double wave_speed(const double u[5], double gamma) {
 // A wave's time step, cell width and constants, held in scalar registers.  All
 // its octs must be of one box; false when they are not, or when the time step
 // or the cell width is out of range.
-RH_DEV double uniform(double x) {
-    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
-                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
-}
-RH_DEV float uniform(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 template <typename T>
 RH_DEV bool constants(const StepArgs& a, int p, double& dt, double& dx, Consts<T>& k) {
     bool ok = true;
@@ -738,50 +915,53 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
     bool ok = constants(a, c.p, dt, dx, k);
     take_cell(u, k, c, ok);
     const double dtdx = uniform(dt / dx), k8 = uniform(dtdx * 0.125);
-    const int E0 = oct_across<0>(lv, c), E1 = oct_across<1>(lv, c), E2 = oct_across<2>(lv, c);
-    const Across n[3] = {across<0>(m, lv, c, E0), across<1>(m, lv, c, E1), across<2>(m, lv, c, E2)};
-    double fs[5], w[5], un[5], wn[5];
-    T ws[5];
-    load5(m, m.uold, n[0].X, u);
-    load5(m, m.uold, n[0].X2, w);
-    auto pass = [&](auto dc) {
-        constexpr int D = decltype(dc)::value;
-        DimFlux<T> f;
-        auto next = [&]() {
-            if constexpr (D < 2) {
-                load5(m, m.uold, n[D + 1].X, un);
-                load5(m, m.uold, n[D + 1].X2, wn);
+    if (__builtin_expect(all_lanes(ok), 1)) {
+        const int E0 = oct_across<0>(lv, c), E1 = oct_across<1>(lv, c), E2 = oct_across<2>(lv, c);
+        const Across n[3] = {across<0>(m, lv, c, E0), across<1>(m, lv, c, E1), across<2>(m, lv, c, E2)};
+        double fs[5], w[5], un[5], wn[5];
+        T ws[5];
+        load5(m, m.uold, n[0].X, u);
+        load5(m, m.uold, n[0].X2, w);
+        auto pass = [&](auto dc) {
+            constexpr int D = decltype(dc)::value;
+            DimFlux<T> f;
+            auto next = [&]() {
+                if constexpr (D < 2) {
+                    load5(m, m.uold, n[D + 1].X, un);
+                    load5(m, m.uold, n[D + 1].X2, wn);
+                } else {
+                    load5(m, a.pre, c.cC, un);
+                }
+            };
+            dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n[D], u, w, k8, ok, f, ws,
+                                             s_x, t, next);
+            copy5(un, u);
+            copy5(wn, w);
+            const bool par = (c.ic0 >> D) & 1;
+            if constexpr (D < 2)
+#pragma unroll
+                for (int iv = 0; iv < 5; ++iv) s_x[15 + 5 * D + iv][t] = ws[iv];
+            if constexpr (D == 0) {
+                // From 0 the order of the two faces does not matter.
+#pragma unroll
+                for (int i = 0; i < 5; ++i) {
+                    const double v = (double)f.Fe[i] - (double)f.Fi[i];
+                    fs[rot<D>(i)] = i == 1 ? flip(v, par ? (int)0x80000000 : 0) : v;
+                }
             } else {
-                load5(m, a.pre, c.cC, un);
+                add_own<D>(fs, f, par);
             }
         };
-        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n[D], u, w, k8, ok, f, ws,
-                                         s_x, t, next);
-        copy5(un, u);
-        copy5(wn, w);
-        const bool par = (c.ic0 >> D) & 1;
-        if constexpr (D < 2)
-#pragma unroll
-            for (int iv = 0; iv < 5; ++iv) s_x[15 + 5 * D + iv][t] = ws[iv];
-        if constexpr (D == 0) {
-            // From 0 the order of the two faces does not matter.
-#pragma unroll
-            for (int i = 0; i < 5; ++i) {
-                const double v = (double)f.Fe[i] - (double)f.Fi[i];
-                fs[rot<D>(i)] = i == 1 ? flip(v, par ? (int)0x80000000 : 0) : v;
-            }
-        } else {
-            add_own<D>(fs, f, par);
-        }
-    };
-    pass(std::integral_constant<int, 0>{});
-    pass(std::integral_constant<int, 1>{});
-    pass(std::integral_constant<int, 2>{});
-    const int key[3] = {n[0].E * 4, n[1].E * 4 + 1, n[2].E * 4 + 2};
-    ok = ok & applies_to<T>(u, fs);
-    apply(u, fs, ws, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
+        pass(std::integral_constant<int, 0>{});
+        if (__builtin_expect(all_lanes(ok), 1)) pass(std::integral_constant<int, 1>{});
+        if (__builtin_expect(all_lanes(ok), 1)) pass(std::integral_constant<int, 2>{});
+        const int key[3] = {n[0].E * 4, n[1].E * 4 + 1, n[2].E * 4 + 2};
+        ok = ok & applies_to<T>(u, fs);
+        if (__builtin_expect(all_lanes(ok), 1))
+            apply(u, fs, ws, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
+    }
     if (__builtin_expect(!all_lanes(ok), 0)) {
-        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, dt, dx, u);
+        general_wave<R, MIXED, EXACT, SHARED>(launch_args(), shared_rows(s_x), praw, t, dt, dx, u);
     }
     finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a);
 }
@@ -789,10 +969,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
 template <int R, bool MIXED, bool EXACT, bool SHARED>
 __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_DIMS_WAVES_F : RH_DIMS_WAVES, 8))) void k_step_dims(StepArgs a) {
     using T = typename std::conditional<MIXED, float, double>::type;
-    // Contributions of X and S per dimension, own fluxes of dimensions 1 and 2
-    // for the first wave, the oct across per dimension, range votes.
+    // Contributions of X and S per dimension, own fluxes for the first
+    // wave, the oct across per dimension, range votes.
     __shared__ T s_x[30][64];
-    __shared__ T s_o[20][64];
+    __shared__ T s_o[30][64];
     __shared__ int s_key[2][64];
     __shared__ int s_bad[3];
     const MeshDev& m = a.m;
@@ -809,38 +989,56 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
     take_cell(u, k, c, ok);
     const double dtdx = uniform(dt / dx), k8 = uniform(dtdx * 0.125);
     double fs[5];
-    int key[3];
+    int key0 = 0;
+    // Rows of s_o: own fluxes of dimensions 1 and 2, then of dimension 0 where
+    // they come from the general form.
+    constexpr int OWN[3] = {20, 0, 10};
+    auto own = [&](auto dc, DimFlux<T>& f) {
+        constexpr int D = decltype(dc)::value;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            f.Fe[i] = s_o[OWN[D] + i][t];
+            f.Fi[i] = s_o[OWN[D] + 5 + i][t];
+        }
+    };
     auto pass = [&](auto dc) {
         constexpr int D = decltype(dc)::value;
         DimFlux<T> f;
-        T ws[5];
-        double x[5], w[5];
-        const Across n = across<D>(m, lv, c, oct_across<D>(lv, c));
-        load5(m, m.uold, n.X, x);
-        load5(m, m.uold, n.X2, w);
-        dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n, x, w, k8, ok, f, ws, s_x, t,
-                                         [] {});
-        const int kd = n.E * 4 + D;
-        const bool par = (c.ic0 >> D) & 1;
-#pragma unroll
-        for (int iv = 0; iv < 5; ++iv) s_x[15 + 5 * D + iv][t] = ws[iv];
-        if constexpr (D == 0) {
-            key[0] = kd;
+        if (__builtin_expect(all_lanes(ok), 1)) {
+            T ws[5];
+            double x[5], w[5];
+            const Across n = across<D>(m, lv, c, oct_across<D>(lv, c));
+            load5(m, m.uold, n.X, x);
+            load5(m, m.uold, n.X2, w);
+            dim_pass<R, T, EXACT, SHARED, D>(m, lv, a.gp.slope_type, a.gp.interpol_type, k, c, n, x, w, k8, ok, f, ws,
+                                             s_x, t, [] {});
+            const int kd = n.E * 4 + D;
+            if constexpr (D == 0) key0 = kd;
+            else s_key[D - 1][t] = kd;
 #pragma unroll
             for (int i = 0; i < 5; ++i) {
-                const double v = (double)f.Fe[i] - (double)f.Fi[i];
-                fs[rot<D>(i)] = i == 1 ? flip(v, par ? (int)0x80000000 : 0) : v;
-            }
-        } else {
-            s_key[D - 1][t] = kd;
-#pragma unroll
-            for (int i = 0; i < 5; ++i) {
-                s_o[10 * (D - 1) + i][t] = f.Fe[i];
-                s_o[10 * (D - 1) + 5 + i][t] = f.Fi[i];
+                s_x[15 + 5 * D + i][t] = ws[i];
+                if constexpr (D > 0) {
+                    s_o[OWN[D] + i][t] = f.Fe[i];
+                    s_o[OWN[D] + 5 + i][t] = f.Fi[i];
+                }
             }
         }
         const bool bad = !all_lanes(ok);  // every lane votes
         if (t == 0) s_bad[D] = bad;
+        if (__builtin_expect(bad, 0)) {
+            general_one_dim<R, MIXED, EXACT, SHARED>(launch_args(), shared_rows(s_x), shared_rows(s_o + OWN[D]), D, praw,
+                                                     t, dt, dx);
+            if constexpr (D == 0) own(dc, f);
+        }
+        if constexpr (D == 0) {
+            const bool par = c.ic0 & 1;
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                const double v = (double)f.Fe[i] - (double)f.Fi[i];
+                fs[i] = i == 1 ? flip(v, par ? (int)0x80000000 : 0) : v;
+            }
+        }
     };
     if (d == 0) pass(std::integral_constant<int, 0>{});
     else if (d == 1) pass(std::integral_constant<int, 1>{});
@@ -850,24 +1048,24 @@ __global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_
     auto other = [&](auto dc) {
         constexpr int D = decltype(dc)::value;
         DimFlux<T> f;
-        key[D] = s_key[D - 1][t];
-#pragma unroll
-        for (int i = 0; i < 5; ++i) {
-            f.Fe[i] = s_o[10 * (D - 1) + i][t];
-            f.Fi[i] = s_o[10 * (D - 1) + 5 + i][t];
-        }
+        own(dc, f);
         add_own<D>(fs, f, (c.ic0 >> D) & 1);
     };
     other(std::integral_constant<int, 1>{});
     other(std::integral_constant<int, 2>{});
-    T ws2[5];
-#pragma unroll
-    for (int iv = 0; iv < 5; ++iv) ws2[iv] = s_x[25 + iv][t];
     load5(m, a.pre, c.cC, u);
     ok = applies_to<T>(u, fs) && !(s_bad[0] | s_bad[1] | s_bad[2]);
-    apply(u, fs, ws2, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
-    if (__builtin_expect(!all_lanes(ok), 0)) {
-        if (c.leaf) general_cell<R, MIXED>(a, c.p, c.ic0, c.cC, s_x, t, dt, dx, u);
+    if (__builtin_expect(all_lanes(ok), 1)) {
+        T ws2[5];
+#pragma unroll
+        for (int iv = 0; iv < 5; ++iv) ws2[iv] = s_x[25 + iv][t];
+        const int key[3] = {key0, s_key[0][t], s_key[1][t]};
+        apply(u, fs, ws2, s_x, key, c.p, c.ic0, t, dtdx, a.gp, uniform(fast::recip(a.gp.gm1)));
+    } else {
+        State5 f;
+        copy5(fs, f.u);
+        const State5 s = general_sum<MIXED>(launch_args(), shared_rows(s_x), f, praw, t, dt, dx);
+        copy5(s.u, u);
     }
     finish(m, lv, a.gp, u, c.leaf, c.cC, c.p, praw - (t >> 3), t, dx, a);
 }
