@@ -88,10 +88,10 @@ struct rh_ctx {
     double* h_interpol = nullptr;
     int interpol_cap = 0;
     // Pinned memory for small results (pinned_small), and whether the
-    // context counts among the users of the staging slots and of the worker
-    // pool (rh_stage.cpp).
+    // context counts among the users of its device's staging slots
+    // (rh_stage.cpp).
     void* h_pin = nullptr;
-    bool stage_user = false, pool_user = false;
+    bool stage_user = false;
     // Godunov kernel variant (rh_set_kernel_variant, rh_autotune); -1: the
     // default, chosen per level by variant_for.
     int variant = -1;

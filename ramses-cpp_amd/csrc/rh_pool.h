@@ -1,7 +1,7 @@
-// rh_pool.h -- the host worker pool of the adaptive driver's flag passes and
-// of long copies.  Host-only (no HIP): the library includes it from rh_amr.cpp
-// and rh_stage.cpp, and the thread-sanitizer test builds it with the host
-// compiler.
+// rh_pool.h -- host worker threads: the pool of the adaptive driver's flag
+// passes, and the class that long copies have their threads from.  Host-only
+// (no HIP): the library includes it from rh_amr.cpp and rh_stage.cpp, and the
+// thread-sanitizer test builds it with the host compiler.
 #pragma once
 #include <algorithm>
 #include <atomic>
@@ -13,20 +13,23 @@
 
 namespace rhi {
 
-// Worker threads shared by every adaptive run of the process and by the
-// contexts that made a long copy: a flag pass is a few hundred microseconds of
-// work, comparable to starting and joining threads, so the passes share one
-// pool instead of spawning their own.  The pool lives while some user does
-// (pool_acquire in rh_amr_create and a context's first long copy, pool_release
-// in rh_amr_destroy and rh_destroy, which joins the workers when the last user
+// Worker threads shared by every adaptive run of the process: a flag pass
+// is a few hundred microseconds of work, comparable to starting and joining
+// threads, so the passes share one pool instead of spawning their own.  The
+// pool lives while some run does (pool_acquire in rh_amr_create,
+// pool_release in rh_amr_destroy, which joins the workers when the last run
 // goes; a pool still alive when the library is unloaded is joined then).
 // run() hands out chunks [k*chunk, (k+1)*chunk) through an atomic counter;
 // the caller works too and returns once every chunk is done.  Passes from
 // different host threads take turns (run_mu_).
 class HostPool {
   public:
+    // Where the system refuses a thread the pool works with those it has.
     explicit HostPool(int nworkers) {
-        for (int i = 0; i < nworkers; ++i) threads_.emplace_back([this] { worker(); });
+        try {
+            for (int i = 0; i < nworkers; ++i) threads_.emplace_back([this] { worker(); });
+        } catch (...) {
+        }
     }
     ~HostPool() {
         {

@@ -1,11 +1,14 @@
 // rh_stage.cpp -- see rh_stage.h.  The slots are shared by the contexts of a
-// process, one set per device: STAGE_SLOTS pieces of pinned memory, allocated
-// by the first copy that needs them and freed with the last context that used
-// them.  Copies of different contexts on one device take turns.
+// process, one set per device: STAGE_SLOTS pieces of pinned memory and a thread
+// for all but one of them, allocated by the first copy that needs them and
+// given back with the last context that used them.  Copies of different
+// contexts on one device take turns; those on different devices, and the
+// worker threads of adaptive runs, do not wait for one another.
 #include "rh_stage.h"
 
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <mutex>
 
 #include "rh_context.h"
@@ -15,7 +18,10 @@ namespace rhi {
 
 namespace {
 
-constexpr int STAGE_SLOTS = 8;
+// Four lanes reach what eight do (96 MB 2.46 ms each way with either), in half
+// the pinned memory and threads that a context alone on its device allocates
+// and gives back; pieces of 1 MB take 3.1 ms.
+constexpr int STAGE_SLOTS = 4;
 constexpr size_t STAGE_PIECE = (size_t)2 << 20;
 constexpr size_t STAGE_LANES = (size_t)10 << 20;
 constexpr size_t STAGE_FEW_RUNS = 4;
@@ -30,6 +36,7 @@ struct Stage {
     std::mutex mu;  // one copy at a time
     char* mem = nullptr;
     Slot slots[STAGE_SLOTS];
+    std::unique_ptr<HostPool> lanes;  // joined before the slots go
     int users = 0;
 };
 
@@ -48,7 +55,8 @@ Stage* stage_of(rh_ctx* c) {
     return s;
 }
 
-// Every slot, in one allocation: freeing eight takes 2 ms longer.
+// Every slot, in one allocation: freeing them one by one takes longer (eight,
+// 2 ms).
 bool ensure_slots(Stage& s) {
     if (!s.mem && hipHostMalloc((void**)&s.mem, STAGE_SLOTS * STAGE_PIECE, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
@@ -110,15 +118,11 @@ int staged(rh_ctx* c, const std::vector<HostRun>& host, char* dev, bool to_host)
     Stage* s = stage_of(c);
     if (!s) return plain(c, host, dev, to_host);
     const size_t npiece = (total + STAGE_PIECE - 1) / STAGE_PIECE;
-    int lanes = (int)std::min<size_t>({npiece, (size_t)STAGE_SLOTS, (size_t)host_threads()});
-    if (lanes > 1 && !c->pool_user) {
-        pool_acquire();
-        c->pool_user = true;
-    }
+    const int most = std::min(STAGE_SLOTS, host_threads());
+    const int lanes = (int)std::min<size_t>(npiece, most);
     std::lock_guard<std::mutex> lk(s->mu);
     if (!ensure_slots(*s)) return plain(c, host, dev, to_host);
-    HostPool* pool = lanes > 1 ? g_pool.load() : nullptr;
-    if (!pool) lanes = 1;
+    if (lanes > 1 && !s->lanes) s->lanes.reset(new HostPool(most - 1));
     hipError_t err[STAGE_SLOTS] = {};
     auto lane = [&](int i) {
         Slot& sl = s->slots[i];
@@ -142,7 +146,7 @@ int staged(rh_ctx* c, const std::vector<HostRun>& host, char* dev, bool to_host)
         err[i] = e;
     };
     if (lanes == 1) lane(0);
-    else pool->run(lanes, lane);
+    else s->lanes->run(lanes, lane);
     for (int i = 0; i < lanes; ++i)
         if (err[i] != hipSuccess) return hip_fail(c, err[i], "staged copy");
     return RH_OK;
@@ -170,6 +174,7 @@ void stage_release(rh_ctx* c) {
         std::lock_guard<std::mutex> lk(g_users_mu);
         Stage& s = g_stages[c->p.device];
         if (--s.users == 0) {
+            s.lanes.reset();
             for (Slot& sl : s.slots) {
                 if (sl.done) (void)hipEventDestroy(sl.done);
                 sl = Slot{};
@@ -179,8 +184,6 @@ void stage_release(rh_ctx* c) {
         }
         c->stage_user = false;
     }
-    if (c->pool_user) pool_release();
-    c->pool_user = false;
 }
 
 }  // namespace rhi

@@ -1,12 +1,16 @@
 // rh_stage.h -- copies between the caller's (pageable) arrays and the device
 // through pinned staging slots.
 //
-// A plain copy of pageable memory runs at 17-18 GB/s here, staged by one
-// thread of the runtime.  Long copies instead move pieces of STAGE_PIECE bytes
-// through pinned slots, several host threads each owning one: a thread queues
-// its piece on the context's stream, waits for it and copies it out while the
-// others' pieces are on the bus (767 MB to the host 44 -> 19 ms, 97 MB 5.4 ->
-// 2.5 ms, 40 MB 2.3 -> 1.1 ms, 12 MB 0.68 -> 0.44 ms).
+// A plain copy of pageable memory runs at 17-18 GB/s to the host here and 27-30
+// to the device, staged by one thread of the runtime.  Long copies instead move
+// pieces of STAGE_PIECE bytes through pinned slots, several host threads each
+// owning one: a thread queues its piece on the context's stream, waits for it
+// and copies it out while the others' pieces are on the bus (to the host 767 MB
+// 43 -> 19 ms, 96 MB 5.5 -> 2.5 ms, 32 MB 1.9 -> 0.9 ms, 12 MB 0.72 -> 0.40 ms;
+// to the device 25 -> 19, 3.3 -> 2.5, 1.07 -> 0.92 and 0.45 -> 0.43 ms).  A
+// context that binds 12 MB, takes a Courant step, reads the state back and goes
+// takes 1.61 ms, slots and threads included, 1.81 with plain copies; one that
+// makes no launch at all pays up to 3 ms for its slots.
 #pragma once
 #include <hip/hip_runtime.h>
 
