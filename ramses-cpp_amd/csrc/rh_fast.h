@@ -3,14 +3,13 @@
 // same operands in the same order, so every value is the same, with the
 // steps left out that cannot matter for a state in range.
 //
-// In range (in_range below, checked per wave on every state a cell's update
-// reads; a wave with a state outside takes the general code) means finite and
-// far from overflow and underflow, so that
+// In range (prim below checks every state a cell's update reads; a wave with a
+// state outside takes the general code) means finite and far from overflow and
+// underflow, so that
 //   * a quotient needs neither the scaling nor the fix-up of the IEEE
 //     division sequence: a reciprocal refined to the last bit (4 instructions)
-//     and a product corrected by its exact remainder (3), which rounds
-//     correctly as IEEE division does; quotients by one divisor share its
-//     reciprocal;
+//     and a product corrected by its exact remainder (3); quotients by one
+//     divisor share its reciprocal;
 //   * a square root needs no scaling (11 instructions instead of 18);
 //   * no operand of a minimum or maximum is a NaN, so v_min/v_max replace
 //     compare-and-select pairs (3 instructions for a double);
@@ -51,9 +50,19 @@ RH_DEV float nonneg(float a) { return smax(a, 0.0f); }
 RH_DEV double signed_as(double a, double s) { return __builtin_copysign(a, s); }
 RH_DEV float signed_as(float a, float s) { return __builtin_copysignf(a, s); }
 
-// Reciprocal (the hardware's, good to 2^-23 at least, times 1 + e + e^2 with
-// its error e: 2^-69 before the last rounding), and a quotient by a divisor
-// whose reciprocal is known (float: the hardware reciprocal, as dv()).
+// Reciprocal (the hardware's, good to 2^-24, times 1 + e + e^2 with its error
+// e: 2^-72 before the last rounding), and a quotient by a divisor whose
+// reciprocal is known (float: the hardware reciprocal, as dv()).
+//
+// Markstein's theorem (IBM J. Res. Dev. 34, 1990): the product corrected by its
+// exact remainder is the correctly rounded quotient where the reciprocal is the
+// correctly rounded one.  unit_quot's is, for every divisor but a significand of
+// all ones, and for that one too where the hardware's is not below it (gfx950
+// returns the correctly rounded reciprocal itself there).  So quotients by a
+// cell's density, whose reciprocal prim takes from unit_quot, round as IEEE
+// division does.  recip's alone misses the last bit for one divisor in 2^17; a
+// quotient by such a divisor differs from IEEE's only next to a midpoint of two
+// doubles, for a handful of its 2^52 dividends.
 RH_DEV double recip(double b) {
     const double y = __builtin_amdgcn_rcp(b);
     const double e = fm(-b, y, 1.0);
@@ -70,16 +79,19 @@ RH_DEV float quot(float a, float, float y) { return a * y; }
 RH_DEV double unit_quot(double b, double y) { return fm(fm(-b, y, 1.0), y, y); }
 RH_DEV float unit_quot(float, float y) { return y; }
 
-// Square root of a value of at least 1e-20.
+// Square root of a value of at least 1e-20: a Newton step for half the
+// reciprocal root h (from the hardware's, good to 2^-24, to 2^-47), then the
+// root 2x*h corrected twice by its exact remainder times h, as Markstein's
+// quotients are: the first leaves it within an ulp, the second within 2^-47 ulp
+// of the root before it is rounded.  A root lies that close to a midpoint of
+// two doubles only for some 1,400 significands; for those, and for 2 10^10
+// others, gfx950 gives the correctly rounded root.
 RH_DEV double root(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double s0 = x * y, h0 = y * 0.5;
-    const double r0 = fm(-h0, s0, 0.5);
-    const double s1 = fm(s0, r0, s0), h1 = fm(h0, r0, h0);
-    const double d0 = fm(-s1, s1, x);
-    const double s2 = fm(d0, h1, s1);
-    const double d1 = fm(-s2, s2, x);
-    return fm(d1, h1, s2);
+    const double g = 0.5 * __builtin_amdgcn_rsq(x), xx = x + x;
+    const double h = fm(g, fm(-(xx * g), g, 0.5), g);
+    double s = xx * h;
+    s = fm(fm(-s, s, x), h, s);
+    return fm(fm(-s, s, x), h, s);
 }
 RH_DEV float root(float x) { return __builtin_amdgcn_sqrtf(x); }
 
@@ -98,36 +110,40 @@ template <typename T> struct Consts {
 RH_DEV double e_int(double p, const Consts<double>& k) { return quot(p, k.gm1, k.y_gm1); }
 RH_DEV float e_int(float p, const Consts<float>& k) { return p * k.y_gm1; }
 
-// Upper bound of a state in range (prim).  Within its bounds, and with dt/dx
-// <= 2^20, dt >= 2^-100, dx in [2^-60, 2^60] and gamma - 1 in [2^-10, 64], no
-// FP64 intermediate of the update exceeds 1e290 and none that is rounded falls
-// below the normal numbers where that could show; the smallest difference of
-// two velocities is 2^-453, so products of two differences do not vanish
-// (FP32: see kept).
+// Bounds of a state in range (prim).  Within them, and with dt/dx <= 2^20, dt >=
+// 2^-100, dx in [2^-60, 2^60] and gamma - 1 in [2^-10, 64], no FP64 intermediate
+// of the update exceeds 1e290 and none that is rounded falls below the normal
+// numbers where that could show; the smallest difference of two velocities is
+// 2^-453, so products of two differences do not vanish.  FP32 has less room: its
+// lower bound is higher, products that vanish are handled by kept, and fluxes
+// that overflow are caught by watch.
 constexpr double RANGE_HI = 0x1p50;
+constexpr double RANGE_LO = 1e-10;
+constexpr float RANGE_LO_F = 0x1p-20f;
+constexpr int RANGE_EXP = -400;   // of a velocity other than 0
+constexpr int TINY_EXP_F = -45;  // of an FP32 velocity that kept looks after
 
-// Conservative -> primitive (the operations of ctoprim); y = recip(density).
+// Conservative -> primitive (the operations of ctoprim); y = 1/density.
 // ok is cleared when the state is out of range: below the floors (density and
-// internal specific energy t of at least RANGE_LO; then no floor of ctoprim or
-// of the trace's sound speed applies either), too large (s covers the density,
-// t and twice the kinetic specific energy; a NaN or an infinity in any
-// component reaches s), or with a velocity that is tiny but not 0 (frexp's
+// internal specific energy t of at least RANGE_LO or RANGE_LO_F; then no floor
+// of ctoprim or of the trace's sound speed applies either), too large (s covers
+// the density, t and twice the kinetic specific energy; a NaN or an infinity in
+// any component reaches s), or with a velocity that is tiny but not 0 (frexp's
 // exponent of 0 is 0, so a zero velocity passes).  tiny is set for an FP32
 // velocity whose differences' products may vanish.
 RH_DEV void prim(const double u[5], double q[5], double& y, const Consts<double>& k, bool& ok, bool&) {
-    y = recip(u[0]);
-    const double o = unit_quot(u[0], y);
+    y = unit_quot(u[0], recip(u[0]));
     q[0] = u[0];
-    q[1] = u[1] * o;
-    q[2] = u[2] * o;
-    q[3] = u[3] * o;
+    q[1] = u[1] * y;
+    q[2] = u[2] * y;
+    q[3] = u[3] * y;
     const double v2 = (q[1] * q[1] + q[2] * q[2]) + q[3] * q[3];
-    const double t = fm(-0.5, v2, u[4] * o);
+    const double t = fm(-0.5, v2, u[4] * y);
     q[4] = k.gm1 * u[0] * t;
     const double s = (v2 + t) + u[0];
     const int least = min(min(__builtin_amdgcn_frexp_exp(q[1]), __builtin_amdgcn_frexp_exp(q[2])),
                           __builtin_amdgcn_frexp_exp(q[3]));
-    ok = ok & (s < RANGE_HI) & (mn(u[0], t) >= 1e-10) & (least > -400);
+    ok = ok & (s < RANGE_HI) & (mn(u[0], t) >= RANGE_LO) & (least > RANGE_EXP);
 }
 RH_DEV void prim(const double ud[5], float q[5], float& y, const Consts<float>& k, bool& ok, bool& tiny) {
     float u[5];
@@ -144,8 +160,8 @@ RH_DEV void prim(const double ud[5], float q[5], float& y, const Consts<float>& 
     const float s = (v2 + t) + u[0];
     const int least = min(min(__builtin_amdgcn_frexp_expf(q[1]), __builtin_amdgcn_frexp_expf(q[2])),
                           __builtin_amdgcn_frexp_expf(q[3]));
-    ok = ok & (s < (float)RANGE_HI) & (mn(u[0], t) >= 0x1p-20f);
-    tiny = tiny | (least <= -45);
+    ok = ok & (s < (float)RANGE_HI) & (mn(u[0], t) >= RANGE_LO_F);
+    tiny = tiny | (least <= TINY_EXP_F);
 }
 
 // Sound speed squared of a trace (its floors: see prim).

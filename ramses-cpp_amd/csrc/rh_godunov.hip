@@ -493,7 +493,7 @@ template <typename T> struct DimFlux {
 template <typename T> struct Cell {
     int p, ic0, lm, cC;
     bool leaf, tiny;  // tiny: see fast::prim
-    T q[5], y, c2;  // primitives in global order, recip(density), trace_c2
+    T q[5], y, c2;  // primitives in global order, 1/density, trace_c2
 };
 
 // A contribution to a cell is -((dtdx*sign)*F)*0.125 with the neighbour's flux
@@ -1093,8 +1093,6 @@ template <int R> void launch_step(bool mixed, bool dims, const StepArgs& a, hipS
     if (mixed) launch_prec<R, true>(dims, a, stream);
     else launch_prec<R, false>(dims, a, stream);
 }
-#ifndef RH_PROBE
 template void launch_step<RH_RIEMANN>(bool, bool, const StepArgs&, hipStream_t);
-#endif
 
 }  // namespace rh
