@@ -32,23 +32,14 @@
 #include "rh_fast.h"
 #include "rh_godunov.h"
 
-// Waves per SIMD asked for (registers per lane: 256 / 168 / 128 at 2 / 3 / 4).
-#ifndef RH_OCT_WAVES
-#define RH_OCT_WAVES 3
-#endif
-#ifndef RH_OCT_WAVES_F
-#define RH_OCT_WAVES_F 3
-#endif
-#ifndef RH_DIMS_WAVES
-#define RH_DIMS_WAVES 3
-#endif
-#ifndef RH_DIMS_WAVES_F
-#define RH_DIMS_WAVES_F 3
-#endif
-
 namespace rh {
 
 namespace {
+
+// Waves per SIMD asked for (registers per lane: 168 / 128 at 3 / 4).  The mixed
+// k_step_dims needs 120 with its general form out of line; at three waves that
+// took 163 and the launch 1.95 ms at 2^21 octs instead of 1.78.
+constexpr int OCT_WAVES = 3, DIMS_WAVES = 3, DIMS_WAVES_F = 4;
 
 using fast::all_lanes;
 using fast::any_lane;
@@ -900,7 +891,7 @@ template <typename T> RH_DEV void take_cell(const double u[5], const Consts<T>& 
 }
 
 template <int R, bool MIXED, bool EXACT, bool SHARED>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_OCT_WAVES_F : RH_OCT_WAVES, 8))) void k_step_oct(StepArgs a) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(OCT_WAVES, 8))) void k_step_oct(StepArgs a) {
     using T = typename std::conditional<MIXED, float, double>::type;
     __shared__ T s_x[25][64];
     const MeshDev& m = a.m;
@@ -967,7 +958,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_O
 }
 
 template <int R, bool MIXED, bool EXACT, bool SHARED>
-__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? RH_DIMS_WAVES_F : RH_DIMS_WAVES, 8))) void k_step_dims(StepArgs a) {
+__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(MIXED ? DIMS_WAVES_F : DIMS_WAVES, 8))) void k_step_dims(StepArgs a) {
     using T = typename std::conditional<MIXED, float, double>::type;
     // Contributions of X and S per dimension, own fluxes for the first
     // wave, the oct across per dimension, range votes.
