@@ -46,17 +46,18 @@ BYTES_PER_CELL_UPDATE = 80  # read uold (5 x FP64) + write unew (5 x FP64)
 # kernel sources it was measured on (KERNEL_SOURCES); a build whose sources
 # hash differently reports null instead of a stale figure.
 KERNEL_SOURCES = ["ramses-cpp_amd/csrc/rh_hydro.hip", "ramses-cpp_amd/csrc/rh_godunov.hip",
-                  "ramses-cpp_amd/csrc/rh_fast.h", "ramses-cpp_amd/csrc/rh_device.h",
-                  "ramses-cpp_amd/csrc/rh_physics.h", "ramses-cpp_amd/csrc/rh_kernels.h", "ramses-cpp_amd/Makefile"]
+                  "ramses-cpp_amd/csrc/rh_godunov.h", "ramses-cpp_amd/csrc/rh_fast.h",
+                  "ramses-cpp_amd/csrc/rh_device.h", "ramses-cpp_amd/csrc/rh_physics.h",
+                  "ramses-cpp_amd/csrc/rh_kernels.h", "ramses-cpp_amd/Makefile"]
 PROFILED = {
-    (9, "hllc", 1, 2, "fp64"): {"sources": "fb7f48747b7e9448", "traffic": 2187115066,
-                                "valu": {"busy": 0.799, "insts_per_cell": 2689.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 6, "fp64"): {"sources": "fb7f48747b7e9448", "traffic": 2175554237,
-                                "valu": {"busy": 0.635, "insts_per_cell": 2920.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 2, "mixed"): {"sources": "fb7f48747b7e9448", "traffic": 2221442369,
-                                 "valu": {"busy": 0.674, "insts_per_cell": 2148.0, "courant_epilogue": True}},
-    (9, "hllc", 1, 6, "mixed"): {"sources": "fb7f48747b7e9448", "traffic": 2177282211,
-                                 "valu": {"busy": 0.648, "insts_per_cell": 2422.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 2, "fp64"): {"sources": "35469fc05691aa54", "traffic": 2190277889,
+                                "valu": {"busy": 0.791, "insts_per_cell": 2701.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 6, "fp64"): {"sources": "35469fc05691aa54", "traffic": 2176190115,
+                                "valu": {"busy": 0.643, "insts_per_cell": 2988.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 2, "mixed"): {"sources": "35469fc05691aa54", "traffic": 2195067668,
+                                 "valu": {"busy": 0.685, "insts_per_cell": 2199.0, "courant_epilogue": True}},
+    (9, "hllc", 1, 6, "mixed"): {"sources": "35469fc05691aa54", "traffic": 2170361214,
+                                 "valu": {"busy": 0.661, "insts_per_cell": 2466.0, "courant_epilogue": True}},
 }
 
 

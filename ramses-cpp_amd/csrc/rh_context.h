@@ -170,11 +170,11 @@ void unbind(rh_ctx* c);
 // The Godunov kernel variant of a launch on lv: the context's when one is
 // set, else the measured default.  Below AUTO_DIMS_MAX_OCTS octs one wave
 // per dimension (variant 6): the level does not fill the GPU and its update
-// takes as long as one wave does (512 octs 10.0 against 13.9 us, 4,096 octs
-// 12.9 against 15.3; mixed 9.1 against 11.8, 10.8 against 13.4).  From there
+// takes as long as one wave does (512 octs 10.4 against 13.7 us, 4,096 octs
+// 12.1 against 14.6; mixed 9.9 against 12.2, 11.4 against 13.6).  From there
 // on one wave per 8 octs (variant 2), which executes fewer instructions
-// (32,768 octs 38.6 against 43.1 us, 2^21 octs 1.90 against 2.23 ms; mixed
-// 29.7 against 34.0, 1.54 against 1.91).  Where the step kernels do not take
+// (32,768 octs 35.3 against 43.4 us, 2^21 octs 1.72 against 2.2 ms; mixed
+// 30.1 against 33.1, 1.46 against 1.70).  Where the step kernels do not take
 // the configuration, variant 6 stays ahead in the FP64 form at every size
 // (3.46 against 3.54 ms).
 constexpr int AUTO_DIMS_MAX_OCTS = 16384;

@@ -6,24 +6,25 @@
 //
 // The eight cells of an oct sit in eight adjacent lanes, a lane's sibling
 // along dimension d is lane ^ (1 << d).  Both kernels run dim_pass, which
-// computes one dimension of a cell's update in the frame of rh_fast.h, and
-// general_cell for the octs of a wave in which some state is out of that
-// frame's range.
+// computes one dimension of a cell's update in the frame of rh_fast.h, and for
+// the waves in which some state is out of that frame's range the general form
+// (general_dim).
 //
-// Bound: the vector ALU, 79 % (FP64) and 68 % (mixed) busy at the 1.9-2.2 GHz
-// that these launches run at.  An HLLC/MinMod update executes 2,545 VALU
-// instructions per cell in the FP64 form and 2,015 in the mixed form, and 150
-// more for the next step's Courant candidate (the kernels of rh_hydro.hip,
+// Bound: the vector ALU, 78-79 % (FP64) and 65-69 % (mixed) busy at the
+// 1.8-2.2 GHz that these launches run at.  An HLLC/MinMod update executes 2,552
+// VALU instructions per cell in the FP64 form and 2,050 in the mixed form, and
+// 149 more for the next step's Courant candidate (the kernels of rh_hydro.hip,
 // which select each operand by a cell's place in its oct, round every division
 // separately and trace own and ghost states apart: 5,747 and 3,779, and
 // 180-195); HBM traffic is a quarter of what the memory delivers.  At 2^21
-// octs (256^3 cells) a launch takes 1.71-1.75 ms in the FP64 form and 1.43-1.45
-// ms in the mixed form, against 3.48 and 2.09 ms; at 512 octs 10.0 and 9.1 us
-// against 13.6 and 12.9 us (k_step_dims).
+// octs (256^3 cells) a launch takes 1.69-1.75 ms in the FP64 form and 1.45-1.47
+// ms in the mixed form, against 3.48 and 2.09 ms; at 512 octs 9.4 and 9.2 us
+// against 12.8 and 12.1 us (k_step_dims).
 // Registers: three waves per SIMD (168 per lane).  Two waves took 2.04 ms
 // against 1.90 (FP64, an earlier order of the code), four waves 1.61 against
 // 1.49 (mixed, 24 bytes spilled): a spill is written through to memory for
-// every wave, so what the update keeps per lane is arranged to need none.
+// every wave, so what the ordinary update keeps per lane is arranged to need
+// none (the general form's 180-220 bytes are touched by its waves only).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
